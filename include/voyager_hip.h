@@ -340,6 +340,26 @@ int vh_gemm_mx8_f16(const uint16_t* x, const int32_t* ex, const uint16_t* w, con
                     int64_t N, int64_t K, const vh_epilogue* epi, void* y, int64_t ldy, float* part,
                     int64_t part_bytes, int32_t splits, int32_t tile, vh_stream_t stream);
 
+/* A lowered FP8 site at decode sizes in one launch: quantize(x, x_scale,
+ * qmap=fp8_e4m3) (ops/quantized.py:449-515) of at most 8 bfloat16 rows x
+ * [M, K] (row pitch ldx elements, 16-byte aligned rows) and linear +
+ * dequantize (quantization/quantize_pt2e.py:538-600) against the E4M3 bytes w
+ * [N, K] (row pitch ldw bytes, 16-byte aligned rows), K % 16 == 0; the
+ * epilogue is EPI_ROUND_SCALE.  The codes it multiplies are vh_quantize's. */
+int vh_linear_fp8_rows8(const uint16_t* x, int64_t ldx, const void* x_scale, int32_t x_scale_dtype,
+                        const uint8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K, const vh_epilogue* epi,
+                        void* y, int64_t ldy, vh_stream_t stream);
+
+/* A lowered MX-int8 site at decode sizes in one launch: quantize_mx(x, int8,
+ * [-1], 16, 127, power-of-two scales) (ops/quantized.py:1070-1115) of at most
+ * 8 bfloat16 rows and linear_mx (:651-723) against int8 codes w [N, K] with
+ * one scale byte per 16 (w_scale [N, K / 16], row pitch ldws, 4-byte aligned
+ * rows; scale = 2**(byte - w_bias), w_bias in [128, 133]); EPI_PLAIN.  Both
+ * operands enter the bf16 MFMA as code * 2**e, exactly. */
+int vh_linear_mxint8_rows8(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t ldw, const uint8_t* w_scale,
+                           int64_t ldws, int32_t w_bias, int64_t M, int64_t N, int64_t K, const vh_epilogue* epi,
+                           void* y, int64_t ldy, vh_stream_t stream);
+
 int vh_pack_nf4(const uint8_t* codes, int64_t N, int64_t K, uint8_t* out, vh_stream_t stream);
 
 /* y[M, N] = sum over blocks b of s_x[m, b] * s_w[n, b] * sum_k Lx[m, k] Lw[n, k]

@@ -800,8 +800,12 @@ extern "C" int vh_quantize(const void* x, int32_t x_dtype, const int64_t* shape,
           return (int)VH_EINVAL;  // unreachable: checked by packable()
         } else if constexpr (K == K_E4M3) {
           // 4 groups per thread up to 2^21 groups, 8 beyond (measured best for
-          // the 16.8 MB and 58.7 MB inputs)
-          if (nvec <= (1ll << 21)) {
+          // the 16.8 MB and 58.7 MB inputs); one up to 2^16, where four leave
+          // CUs idle (16 x 4096 in a graph: 3.0 us with four, 2.6 with one)
+          if (nvec <= (1ll << 16)) {
+            hipLaunchKernelGGL(k_quantize_e4m3_pt<1>, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, st,
+                               (const uint16_t*)x, nvec, sp.ptr, sp.dtype, (uint8_t*)out);
+          } else if (nvec <= (1ll << 21)) {
             hipLaunchKernelGGL(k_quantize_e4m3_pt<4>, dim3((unsigned)((nvec + 1023) / 1024)), dim3(256), 0, st,
                                (const uint16_t*)x, nvec, sp.ptr, sp.dtype, (uint8_t*)out);
           } else {

@@ -22,7 +22,9 @@
 #include <cstring>
 
 #include "vh_device.h"
+#include "vh_epilogue.h"
 #include "vh_host.h"
+#include "vh_skinny.h"
 
 namespace {
 
@@ -173,11 +175,6 @@ __host__ __device__ inline bool lds_epilogue_ok(const void* C, int out_dtype, in
 __host__ __device__ inline bool f8dl_epilogue_ok(const void* C, int out_dtype, int64_t ldc, int64_t N) {
   if (out_dtype == VH_F32) return ((uintptr_t)C % 16) == 0 && (ldc % 4) == 0;
   return lds_epilogue_ok(C, out_dtype, ldc, N);
-}
-
-__device__ __forceinline__ float epi_scale(const vh_epilogue& e) {
-  if (!e.scale) return 1.0f;
-  return e.scale_dtype == VH_BF16 ? bf2f(*(const uint16_t*)e.scale) : *(const float*)e.scale;
 }
 
 // Bytes of the direct-to-LDS kernel's bf16 epilogue staging (padded rows);
@@ -345,23 +342,6 @@ __device__ __forceinline__ void store_tile_lds_t(const GemmArgs& g, f32x16 (&acc
     const uint4 v = *(const uint4*)(ct + row * PITCH + ch * 8);
     if (grow < g.M && gcol < g.N) *(uint4*)((uint16_t*)g.C + grow * g.ldc + gcol) = v;
   }
-}
-
-__device__ __forceinline__ float epi_bias(const vh_epilogue& e, int64_t col) {
-  if (!e.bias) return 0.0f;
-  return e.bias_dtype == VH_BF16 ? bf2f(((const uint16_t*)e.bias)[col]) : ((const float*)e.bias)[col];
-}
-
-// The epilogue of one fp32 accumulator (sc = epi_scale, bias = epi_bias).
-__device__ __forceinline__ float epi_value(const vh_epilogue& e, float v, float sc, float bias) {
-  if (e.mode == EPI_ROUND_SCALE) {
-    // dequantize(linear(xq, wq), s): the GEMM rounds to bf16, then the bf16
-    // product with the scale rounds again.
-    return rbf(rbf(v) * sc);
-  }
-  if (e.scale) v = v * sc;
-  if (e.bias) v = v + bias;
-  return v;
 }
 
 // Element-wise stores (f32 output, or bf16 rows the LDS path cannot take).
@@ -2175,6 +2155,7 @@ constexpr int FAM_STAGED = 1;       // k_gemm: register-staged, decodes in stagi
 constexpr int FAM_DIRECT_FP8 = 2;   // k_gemm_f8dl, E4M3 operands
 constexpr int FAM_DIRECT_BF16 = 3;  // k_gemm_f8dl, bf16 operands
 constexpr int FAM_MXI8 = 4;         // k_gemm_mxi8 / k_gemm_mxi8_ws (+ k_split_reduce)
+constexpr int FAM_SKINNY = 5;       // k_skinny: at most 64 rows
 
 struct Plan {
   int family, tile, splits;
@@ -2206,6 +2187,7 @@ Plan plan_gemm(const vh_gemm_desc* d) {
   auto tiles = [&](int bm, int bn) { return ((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn) * batch; };
   const bool fp8 = d->a_fmt == OP_FP8;
   const bool dl_ok = f8dl_epilogue_ok(d->C, d->epi.out_dtype, d->ldc, d->N);
+  if (vh::skinny_fits(d)) return {FAM_SKINNY, 0, 1};
   // Register-staged kernel (bf16, MX-int8 and posit8 operands; fp8 when the
   // LDS epilogue does not apply).  Measured on MI355X at M = 2048 with fp8
   // data (K in {4096, 14336}, N in {1024, 4096, 14336}): 8-wave blocks (two
@@ -2340,6 +2322,7 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
   VH_REQUIRE(batch < 65536, "vh_gemm: batch too large");
   hipStream_t st = vh::as_stream(stream);
   const Plan p = plan_gemm(d);
+  if (p.family == FAM_SKINNY) return vh::skinny_gemm(d, stream);
   if (p.family == FAM_DIRECT_FP8) {
     switch (p.tile) {
       case 20: return launch_f8dl<256, 256, 4, 64>(g, batch, st);
@@ -2413,7 +2396,7 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
 }
 
 extern "C" int64_t vh_gemm_workspace_bytes(const vh_gemm_desc* d) {
-  if (!d) return 0;
+  if (!d || vh::skinny_fits(d)) return 0;
   int cfg, splits;
   mxi8_plan(d, cfg, splits);
   return cfg ? mxi8_workspace(d, splits) : 0;

@@ -140,6 +140,10 @@ _SIGNATURES = {
     "vh_gemm_plan": ([_P, ctypes.POINTER(_I32), ctypes.POINTER(_I32), ctypes.POINTER(_I32)], _I32),
     "vh_quantize_mx_rows16": ([_P, _I32, _I64, _I64, _I64, ctypes.c_float, ctypes.POINTER(Format),
                                ctypes.POINTER(Format), _P, _P, _P, _P], _I32),
+    # x, ldx, x_scale, x_scale_dtype, w, ldw, M, N, K, epilogue*, y, ldy, stream
+    "vh_linear_fp8_rows8": ([_P, _I64, _P, _I32, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _P], _I32),
+    # x, ldx, w, ldw, w_scale, ldws, w_bias, M, N, K, epilogue*, y, ldy, stream
+    "vh_linear_mxint8_rows8": ([_P, _I64, _P, _I64, _P, _I64, _I32, _I64, _I64, _I64, _P, _P, _I64, _P], _I32),
     "vh_pack_nf4": ([_P, _I64, _I64, _P, _P], _I32),
     # x_levels, x_scale, M, w_packed, w_scale, w_scale_fmt, levels16 (host), N, K, epilogue*, y, stream
     "vh_gemv_nf4": ([_P, _P, _I64, _P, _P, ctypes.POINTER(Format), _P, _I64, _I64, _P, _P, _P], _I32),

@@ -58,7 +58,7 @@ class GemmDesc(ctypes.Structure):
     ]
 
 
-FAMILY_STAGED, FAMILY_DIRECT_FP8, FAMILY_DIRECT_BF16, FAMILY_MXI8 = 1, 2, 3, 4
+FAMILY_STAGED, FAMILY_DIRECT_FP8, FAMILY_DIRECT_BF16, FAMILY_MXI8, FAMILY_SKINNY = 1, 2, 3, 4, 5
 
 #: When set to a list, every ``vh_gemm`` launch appends ``(family, tile,
 #: splits, M, N, K)`` of the kernel it runs (``vh_gemm_plan``), so tests can
@@ -320,6 +320,44 @@ def linear_fp8(xq: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, out: Opt
     d.tile_hint = tile_hint
     d.epi = _epilogue(EPI_ROUND_SCALE, torch.bfloat16, scale)
     run(d, xq.device)
+    return out
+
+
+def linear_fp8_rows8(x: torch.Tensor, x_scale: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+    """``linear_fp8(quantize_packed(x, x_scale, fp8_e4m3), wq, scale)`` of at
+    most 8 bf16 rows ``x`` in one launch, on the same codes."""
+    M, K = x.shape
+    N = wq.shape[0]
+    x = x.contiguous()
+    if wq.shape[1] != K or wq.element_size() != 1:
+        raise RuntimeError("linear_fp8_rows8: the weight must hold one-byte codes of the activation's columns")
+    wq = _rows(wq)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    epi = _epilogue(EPI_ROUND_SCALE, torch.bfloat16, scale)
+    st = load().vh_linear_fp8_rows8(ptr(x), K, ptr(x_scale), dtype_code(x_scale.dtype), ptr(wq),
+                                     wq.stride(0), M, N, K, ctypes.c_void_p(ctypes.addressof(epi)), ptr(out), N,
+                                     ctypes.c_void_p(stream_of(x)))
+    _lib.check(st, "vh_linear_fp8_rows8")
+    return out
+
+
+def linear_mxint8_rows8(x: torch.Tensor, w_codes: torch.Tensor, w_scale: torch.Tensor, bias_w: int,
+                         bias=None) -> torch.Tensor:
+    """``linear_mxint8`` of at most 8 bf16 rows ``x``, quantized in the
+    same launch to the same codes, in blocks of 16."""
+    M, K = x.shape
+    N = w_codes.shape[0]
+    x = x.contiguous()
+    if w_codes.shape[1] != K or w_codes.element_size() != 1:
+        raise RuntimeError("linear_mxint8_rows8: the weight must hold one-byte codes of the activation's columns")
+    w_codes, w_scale = _rows(w_codes), _rows(w_scale)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    bias = _bias_operand(bias)
+    epi = _epilogue(EPI_PLAIN, torch.bfloat16, None, bias)
+    st = load().vh_linear_mxint8_rows8(ptr(x), K, ptr(w_codes), w_codes.stride(0), ptr(w_scale),
+                                        w_scale.stride(0), bias_w, M, N, K, ctypes.c_void_p(ctypes.addressof(epi)),
+                                        ptr(out), N, ctypes.c_void_p(stream_of(x)))
+    _lib.check(st, "vh_linear_mxint8_rows8")
     return out
 
 
