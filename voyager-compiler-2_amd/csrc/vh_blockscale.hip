@@ -17,6 +17,7 @@
 
 #include <cstring>
 
+#include "vh_blockfast.h"
 #include "vh_blockscale.h"
 #include "vh_device.h"
 #include "vh_host.h"
@@ -182,14 +183,12 @@ k_rows(const void* __restrict__ x, int64_t rows, int64_t L, int64_t nblk, int g,
 // plain max and a NaN flag -- the same values, codes and bytes.  Thread
 // layout as k_rows<8>: eight consecutive elements, g = block / 8 lanes per
 // block.
-// IDX: the index type (32-bit when every thread index fits).  REF: the
-// reference form instead of packed bytes -- codes as bf16 values (NaN kept,
-// -0 kept) and the scales as bf16 values, as quantized_ops.quantize_mx
-// returns them.
-template <typename IDX, bool REF>
+// IDX: the index type (32-bit when every thread index fits).
+template <typename IDX>
 __global__ void __launch_bounds__(256)
 k_mx_pot_int_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int64_t nblk, int g, int shift,
-                   int pot_bias, float lo, float hi, void* __restrict__ scale_out, void* __restrict__ codes_out) {
+                   int pot_bias, float lo, float hi, uint8_t* __restrict__ scale_out,
+                   uint8_t* __restrict__ codes_out) {
   const IDX tpr = (IDX)(nblk * g);
   const IDX t = (IDX)blockIdx.x * (IDX)blockDim.x + (IDX)threadIdx.x;
   const int64_t row = (int64_t)(t / tpr);
@@ -234,8 +233,7 @@ k_mx_pot_int_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int6
   const int64_t blk = v / g;
   if (v - blk * g == 0 && blk < nblk) {
     const int byte = inf ? 255 : e + pot_bias;
-    if constexpr (REF) ((uint16_t*)scale_out)[row * nblk + blk] = (uint16_t)f2bf(s);
-    else ((uint8_t*)scale_out)[row * nblk + blk] = (uint8_t)(byte < 0 ? 0 : (byte > 254 && !inf ? 254 : byte));
+    scale_out[row * nblk + blk] = (uint8_t)(byte < 0 ? 0 : (byte > 254 && !inf ? 254 : byte));
   }
   if (!live) return;
   // 1 / s exactly when s is a normal power of two: x * (1 / s) is x / s
@@ -254,18 +252,12 @@ k_mx_pot_int_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int6
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float r = fminf(fmaxf(rintf(q[j]), lo), hi);
-    if constexpr (REF) c[j] = q[j] != q[j] ? 0x7FC0u : f2bf(r);  // an integer: exact in bf16
-    else c[j] = q[j] != q[j] ? 0u : ((uint32_t)(int32_t)r & 0xffu);
+    c[j] = q[j] != q[j] ? 0u : ((uint32_t)(int32_t)r & 0xffu);
   }
-  if constexpr (REF) {
-    *(uint4*)((uint16_t*)codes_out + base) =
-        make_uint4(c[0] | (c[1] << 16), c[2] | (c[3] << 16), c[4] | (c[5] << 16), c[6] | (c[7] << 16));
-  } else {
-    uint2 pk;
-    pk.x = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
-    pk.y = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
-    *(uint2*)((uint8_t*)codes_out + base) = pk;
-  }
+  uint2 pk;
+  pk.x = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
+  pk.y = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
+  *(uint2*)(codes_out + base) = pk;
 }
 
 // quantize_mx with a minifloat scale map to packed codebook indices (a
@@ -466,6 +458,46 @@ int dispatch_scale(const Params& P, F&& fn) {
   return fn(std::integral_constant<int, K_RUNTIME>{});
 }
 
+// The kernels of vh_blockfast.h, for the forms they take: bf16 tensors,
+// 16-byte aligned, of fewer than 2**31 elements, to bf16 codes and scales,
+// where the row kernel's layout holds, or blocks of 16, 32 or 64 along another
+// dimension with a multiple of eight elements inside it.
+bool launch_fast(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block, const Params& P,
+                 void* scale_out, void* zp_out, void* codes_out, bool rows_ok, hipStream_t stream) {
+  auto al = [](const void* p, int n) { return ((uintptr_t)p & (uintptr_t)(n - 1)) == 0; };
+  const int64_t nblk = (L + block - 1) / block;
+  if (!codes_out || !al(x, 16) || !al(codes_out, 16) || outer * nblk * block * inner >= (1ll << 31)) return false;
+  const uint16_t* xp = (const uint16_t*)x;
+  uint16_t *sp = (uint16_t*)scale_out, *zp = (uint16_t*)zp_out, *cp = (uint16_t*)codes_out;
+  if (rows_ok) {
+    const int g = (int)(block / 8);
+    const uint32_t threads = (uint32_t)(outer * nblk * g);
+    return dispatch_fast(P, [&](auto m, auto k, auto s) {
+      constexpr int M = decltype(m)::value, K = decltype(k)::value, S = decltype(s)::value;
+      const dim3 grid((threads + 255) / 256);
+      if (L % block == 0)
+        hipLaunchKernelGGL((k_fast_rows<M, K, S, true>), grid, dim3(256), 0, stream, xp, threads, (uint32_t)L,
+                           make_fast_div(1), g, P, sp, zp, cp);
+      else
+        hipLaunchKernelGGL((k_fast_rows<M, K, S, false>), grid, dim3(256), 0, stream, xp, threads, (uint32_t)L,
+                           make_fast_div((uint32_t)(nblk * g)), g, P, sp, zp, cp);
+    });
+  }
+  if (inner % 8 || (block != 16 && block != 32 && block != 64) || !al(scale_out, 4) || (zp_out && !al(zp_out, 4)))
+    return false;
+  const uint32_t total = (uint32_t)(outer * nblk * (inner / 8));
+  return dispatch_fast(P, [&](auto m, auto k, auto s) {
+    constexpr int M = decltype(m)::value, K = decltype(k)::value, S = decltype(s)::value;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((total + 63) / 64), dim3(256), 0, stream, xp, total, L, inner,
+                         make_fast_div((uint32_t)(inner / 8)), make_fast_div((uint32_t)nblk), P, sp, zp, cp);
+    };
+    if (block == 16) go(k_fast_cols<M, K, S, 4>);
+    else if (block == 32) go(k_fast_cols<M, K, S, 8>);
+    else go(k_fast_cols<M, K, S, 16>);
+  });
+}
+
 int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block, const Params& P,
            void* scale_out, void* zp_out, void* codes_out, hipStream_t stream, const char* what) {
   const int64_t nblk = (L + block - 1) / block;
@@ -482,6 +514,8 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
                            (P.scale_dtype == VH_F32 || P.scale_dtype == VH_U8) && !P.gs && codes_out &&
                            P.has_fmt && kernel_kind(&P.fmt) == K_STEPS && P.fmt.nsteps <= 15 && P.has_sfmt &&
                            kernel_kind(&P.sfmt) == K_MINI;
+  if (!steps_lanes && !lanes_ok && launch_fast(x, outer, L, inner, block, P, scale_out, zp_out, codes_out, rows_ok, stream))
+    return vh::check_launch(what);
   if (steps_lanes) {
     const int64_t threads = outer * L;
     hipLaunchKernelGGL(k_mx_steps_lanes, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
@@ -509,23 +543,14 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
     const bool lean = P.mode != AFFINE && P.cdt == VH_BF16 && P.codes_dtype == VH_U8 && P.scale_dtype == VH_U8 &&
                       !P.code_lut && !P.gs && !P.scale_t16 && codes_out && P.has_fmt;
     const int k0 = P.has_fmt ? kernel_kind(&P.fmt) : (int)K_NONE;
-    // the same with reference-form outputs (bf16 codes and scales)
-    const bool lean_ref = P.mode == MX_POT && P.cdt == VH_BF16 && P.codes_dtype == VH_BF16 &&
-                          P.scale_dtype == VH_BF16 && !P.code_lut && !P.gs && !P.scale_t16 && codes_out &&
-                          P.has_fmt && !P.has_sfmt && k0 == K_INT;
-    if ((lean && P.mode == MX_POT && k0 == K_INT && !P.has_sfmt) || lean_ref) {
-      const bool i32 = blocks * 256 < (1ll << 31);
+    if (lean && P.mode == MX_POT && k0 == K_INT && !P.has_sfmt) {
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)x, outer, L, nblk, g,
-                           P.shift, P.pot_bias, (float)P.fmt.p0, (float)P.fmt.p1, scale_out, codes_out);
+                           P.shift, P.pot_bias, (float)P.fmt.p0, (float)P.fmt.p1, (uint8_t*)scale_out,
+                           (uint8_t*)codes_out);
       };
-      if (lean_ref) {
-        if (i32) go(k_mx_pot_int_rows8<uint32_t, true>);
-        else go(k_mx_pot_int_rows8<int64_t, true>);
-      } else {
-        if (i32) go(k_mx_pot_int_rows8<uint32_t, false>);
-        else go(k_mx_pot_int_rows8<int64_t, false>);
-      }
+      if (blocks * 256 < (1ll << 31)) go(k_mx_pot_int_rows8<uint32_t>);
+      else go(k_mx_pot_int_rows8<int64_t>);
     } else if (lean && P.mode == MX_SCALED && k0 == K_STEPS && P.has_sfmt && kernel_kind(&P.sfmt) == K_MINI) {
       if (P.fmt.nsteps <= 15) {
         if (blocks * 256 < (1ll << 31))

@@ -39,6 +39,23 @@ VH_DEV uint32_t f2bf2_hw(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
+// n / d for 32-bit n and a divisor fixed at launch: the upper half of one
+// product and shifts (Granlund and Montgomery, "Division by invariant
+// integers using multiplication", 1994, fig. 4.1).
+struct FastDiv {
+  uint32_t d, m, s1, s2;
+};
+static inline FastDiv make_fast_div(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32 && (1ull << l) < d) ++l;
+  const uint32_t m = (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1);
+  return FastDiv{d, m, l > 1 ? 1u : l, l > 0 ? l - 1 : 0u};
+}
+VH_DEV uint32_t fast_div(uint32_t n, const FastDiv& f) {
+  const uint32_t t = __umulhi(f.m, n);
+  return (t + ((n - t) >> f.s1)) >> f.s2;
+}
+
 // Streaming accesses that bypass cache residency (the nt bit): each element
 // of a large elementwise op is touched once, so its lines should not evict
 // data that is reused.  Measured from HBM (inputs rotated through more than
