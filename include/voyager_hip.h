@@ -406,6 +406,23 @@ int vh_gemm_nf4(const uint8_t* x_idx, const uint8_t* x_scale, const vh_format* x
  * caller's nonzero *tile / *splits are kept, the splits rounded to whole
  * ranges of 64-element blocks), so the caller can size its workspace. */
 int vh_gemm_nf4_plan(int64_t M, int64_t N, int64_t K, int32_t* tile, int32_t* splits, int64_t* bm);
+/* vh_gemm_nf4 on an activation already decoded to bfloat16 (x [M, K], rows
+ * contiguous: bf16(level * scale), vh_nf4_decode_bf16): the same products,
+ * the weight decoded in registers.  x, the weight, its scales, y and part
+ * 16-byte aligned, ldy % 4 == 0.  splits 0 chooses
+ * (vh_gemm_nf4_bf16_plan); with more than one, float32 partials go to part
+ * as in vh_gemm_nf4. */
+int vh_gemm_nf4_bf16(const uint16_t* x, int64_t M, const uint8_t* w_packed, const uint8_t* w_scale,
+                     const vh_format* w_scale_fmt, const int8_t* levels16, int64_t N, int64_t K,
+                     const vh_epilogue* epi, void* y, int64_t ldy, int32_t splits, float* part,
+                     int64_t part_bytes, vh_stream_t stream);
+int vh_gemm_nf4_bf16_plan(int64_t M, int64_t N, int64_t K, int32_t* splits);
+/* Its activation in one pass: quantize_mx of x [M, K] (bfloat16 rows, blocks
+ * of 64 along K, minifloat scale map, index table of at most 16 levels), out
+ * = bf16(level * scale) -- vh_quantize_mx to index and scale bytes, then
+ * vh_nf4_decode_bf16, bit for bit.  x and out 16-byte aligned. */
+int vh_nf4_quantize_bf16(const uint16_t* x, int64_t M, int64_t K, float quant_max, const vh_format* scale_fmt,
+                         const vh_format* fmt, const int8_t* levels16, uint16_t* out, vh_stream_t stream);
 /* The operands of vh_gemm_nf4 decoded once to bfloat16, for the two-pass
  * prefill (decode, then the bf16 GEMM of vh_gemm): x_out [M, K] =
  * bf16(level[x_idx] * x_scale) and w_out [N, K] the weight's rows likewise,

@@ -264,11 +264,14 @@ k_mx_pot_int_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int6
 // table of at most 15 thresholds: the 16-level codebooks), bf16 rows:
 // block_scale (MX_SCALED, no global scale) and element_code (K_STEPS) for
 // that case restated without their runtime switches -- the same scale
-// codes and indices.  Thread layout as k_rows<8>.
-template <typename IDX>
+// codes and indices.  Thread layout as k_rows<8>.  With DEC, instead of
+// both, the operand they decode to: bf16(level * scale), the level of an
+// index from lvb (level + 128, one byte each).
+template <typename IDX, bool DEC = false>
 __global__ void __launch_bounds__(256)
 k_mx_steps_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int64_t nblk, int g, float quant_max,
-                 vh_format sfmt, vh_format fmt, uint8_t* __restrict__ scale_out, uint8_t* __restrict__ codes_out) {
+                 vh_format sfmt, vh_format fmt, uint8_t* __restrict__ scale_out, uint8_t* __restrict__ codes_out,
+                 uint4 lvb = make_uint4(0u, 0u, 0u, 0u)) {
   __shared__ uint16_t keys[16];
   const IDX tpr = (IDX)(nblk * g);
   const IDX t = (IDX)blockIdx.x * (IDX)blockDim.x + (IDX)threadIdx.x;
@@ -300,10 +303,12 @@ k_mx_steps_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int64_
   float s = div_bf16(hi, quant_max);
   s = rbf(fmt_value_k<K_MINI>(f2bf(s), sfmt, nullptr));
   if (!(s > 0.0f)) s = 1.0f;
-  const int64_t blk = v / g;
-  if (v - blk * g == 0 && blk < nblk) {
-    const uint32_t b = f2bf(s);
-    scale_out[row * nblk + blk] = (uint8_t)fmt_code_k<K_MINI>(b, bf2f(b), sfmt, nullptr);
+  if constexpr (!DEC) {
+    const int64_t blk = v / g;
+    if (v - blk * g == 0 && blk < nblk) {
+      const uint32_t b = f2bf(s);
+      scale_out[row * nblk + blk] = (uint8_t)fmt_code_k<K_MINI>(b, bf2f(b), sfmt, nullptr);
+    }
   }
   if (!live) return;
   uint32_t key[8], pos[8];
@@ -328,7 +333,21 @@ k_mx_steps_rows8(const uint16_t* __restrict__ x, int64_t rows, int64_t L, int64_
   uint2 pk;
   pk.x = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
   pk.y = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
-  *(uint2*)(codes_out + base) = pk;
+  if constexpr (DEC) {
+    // the scale as its code decodes (1 where the map does not hold it)
+    const uint32_t b = f2bf(s);
+    const float sd = fmt_decode(fmt_code_k<K_MINI>(b, bf2f(b), sfmt, nullptr) & 0xffu, sfmt, nullptr);
+    const float nb = -128.0f * sd;
+    uint32_t lbase;
+    asm volatile("v_mov_b32 %0, 0x3020100" : "=v"(lbase));
+    float f[4], h[4];
+    nf4_levels4(lut_lo(pk.x, lbase, lvb), sd, nb, f);
+    nf4_levels4(lut_lo(pk.y, lbase, lvb), sd, nb, h);
+    *(uint4*)((uint16_t*)codes_out + base) =
+        make_uint4(f2bf2_hw(f[0], f[1]), f2bf2_hw(f[2], f[3]), f2bf2_hw(h[0], h[1]), f2bf2_hw(h[2], h[3]));
+  } else {
+    *(uint2*)(codes_out + base) = pk;
+  }
 }
 
 // The same at decode sizes, one element per lane (a block's g lanes reduce
@@ -682,6 +701,27 @@ extern "C" int vh_quantize_mx_rows16(const void* x, int32_t x_dtype, int64_t row
   VH_REQUIRE(L % block == 0, "vh_quantize_mx_rows16: L must be a multiple of block");
   return quantize_mx_impl(x, x_dtype, rows, L, 1, block, quant_max, 0, scale_fmt, nullptr, 0, fmt, scale_out, VH_F32,
                           0, codes_out, VH_U8, code_lut, 1, stream);
+}
+
+extern "C" int vh_nf4_quantize_bf16(const uint16_t* x, int64_t M, int64_t K, float quant_max,
+                                    const vh_format* scale_fmt, const vh_format* fmt, const int8_t* levels16,
+                                    uint16_t* out, vh_stream_t stream) {
+  VH_REQUIRE(x && scale_fmt && fmt && levels16 && out, "vh_nf4_quantize_bf16: null argument");
+  VH_REQUIRE(M >= 1 && K > 0 && K % 64 == 0, "vh_nf4_quantize_bf16: needs K %% 64 == 0");
+  VH_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0, "vh_nf4_quantize_bf16: misaligned operand");
+  VH_REQUIRE(kernel_kind(scale_fmt) == K_MINI, "vh_nf4_quantize_bf16: the scale map must be a minifloat");
+  VH_REQUIRE(fmt->kind == VH_FMT_STEPS && fmt->nsteps >= 0 && fmt->nsteps <= 15 && fmt->nan_level <= 15,
+             "vh_nf4_quantize_bf16: the map must be an index table of at most 16 levels");
+  const int64_t blocks = (M * (K / 8) + 255) / 256;
+  VH_REQUIRE(blocks * 256 < (1ll << 31), "vh_nf4_quantize_bf16: tensor too large");
+  uint8_t lvb[16];
+  for (int v = 0; v < 16; ++v) lvb[v] = (uint8_t)(levels16[v] + 128);
+  uint32_t t[4];
+  memcpy(t, lvb, 16);
+  hipLaunchKernelGGL((k_mx_steps_rows8<uint32_t, true>), dim3((unsigned)blocks), dim3(256), 0, vh::as_stream(stream),
+                     x, M, K, K / 64, 8, quant_max, *scale_fmt, *fmt, nullptr, (uint8_t*)out,
+                     make_uint4(t[0], t[1], t[2], t[3]));
+  return vh::check_launch("vh_nf4_quantize_bf16");
 }
 
 extern "C" int vh_quantize_affine(const void* x, int32_t x_dtype, int64_t outer, int64_t L, int64_t inner,

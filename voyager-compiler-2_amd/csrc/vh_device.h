@@ -381,6 +381,30 @@ VH_DEV uint32_t lut_hi(uint32_t w, uint32_t base, const uint4& lv) {
   return lut16((w >> 4) & 0x07070707u, w >> 5, base, lv.x, lv.y, lv.z, lv.w);
 }
 
+// MXNF4 operands, bf16(level * scale): four biased levels (level + 128, one
+// byte each) times s, nb = -128 s
+VH_DEV void nf4_levels4(uint32_t biased, float s, float nb, float (&f)[4]) {
+  f[0] = fmaf((float)(biased & 0xffu), s, nb);
+  f[1] = fmaf((float)((biased >> 8) & 0xffu), s, nb);
+  f[2] = fmaf((float)((biased >> 16) & 0xffu), s, nb);
+  f[3] = fmaf((float)(biased >> 24), s, nb);
+}
+
+// Sixteen biased levels (four dwords, element order) times s -> 16 bf16.
+VH_DEV void nf4_pack16(const uint32_t (&l)[4], float s, uint4& lo, uint4& hi) {
+  const float nb = -128.0f * s;
+  uint32_t o[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float f[4];
+    nf4_levels4(l[j], s, nb, f);
+    o[2 * j] = f2bf2_hw(f[0], f[1]);
+    o[2 * j + 1] = f2bf2_hw(f[2], f[3]);
+  }
+  lo = make_uint4(o[0], o[1], o[2], o[3]);
+  hi = make_uint4(o[4], o[5], o[6], o[7]);
+}
+
 // Kernels are specialised on the format kind (K_* below) so each instance
 // holds only its own closed form; the runtime-dispatch versions serve the
 // per-block scale maps.

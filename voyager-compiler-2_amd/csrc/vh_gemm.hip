@@ -31,6 +31,7 @@ namespace {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // Exact fp16 operands (vh_gemm_mx8_f16); internal to this file, not a
@@ -1105,6 +1106,15 @@ __device__ __forceinline__ void dma16(const i32x4& rsrc, uint32_t lds, int voff)
   asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff), "s"(rsrc), "{m0}"(lds) : "memory");
 }
 
+// dma16 of lanes 0..31 alone (512 bytes); the whole wave has to be active.
+__device__ __forceinline__ void dma16_half(const i32x4& rsrc, uint32_t lds, int voff) {
+  asm volatile(
+      "s_mov_b32 exec_hi, 0\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds\n\ts_mov_b32 exec_hi, -1"
+      :
+      : "v"(voff), "s"(rsrc), "{m0}"(lds)
+      : "memory");
+}
+
 // Waves per SIMD the direct-to-LDS kernel asks for: one per four waves of
 // its workgroup (at least one).
 constexpr int f8dl_wpe(int nw) { return nw >= 4 ? nw / 4 : 1; }
@@ -1822,29 +1832,6 @@ struct Nf4Args {
   vh_format b_sf;   // the weight's scale map
 };
 
-// four indices (one per byte, 0..15) -> four bf16 pairs' worth of floats
-__device__ __forceinline__ void nf4_levels4(uint32_t biased, float s, float nb, float (&f)[4]) {
-  f[0] = fmaf((float)(biased & 0xffu), s, nb);
-  f[1] = fmaf((float)((biased >> 8) & 0xffu), s, nb);
-  f[2] = fmaf((float)((biased >> 16) & 0xffu), s, nb);
-  f[3] = fmaf((float)(biased >> 24), s, nb);
-}
-
-// Sixteen biased levels (four dwords, element order) times s -> 16 bf16.
-__device__ __forceinline__ void nf4_pack16(const uint32_t (&l)[4], float s, uint4& lo, uint4& hi) {
-  const float nb = -128.0f * s;
-  uint32_t o[8];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float f[4];
-    nf4_levels4(l[j], s, nb, f);
-    o[2 * j] = f2bf2_hw(f[0], f[1]);
-    o[2 * j + 1] = f2bf2_hw(f[2], f[3]);
-  }
-  lo = make_uint4(o[0], o[1], o[2], o[3]);
-  hi = make_uint4(o[4], o[5], o[6], o[7]);
-}
-
 template <int BM, int BN, int WM, int WN, int P>
 __global__ void __launch_bounds__(WM * WN * 64) k_gemm_nf4(GemmArgs g, Nf4Args q, int kcs, float* __restrict__ part) {
   constexpr int NT = WM * WN * 64;
@@ -2046,6 +2033,318 @@ int launch_nf4(GemmArgs g, const Nf4Args& q, int splits, float* part, hipStream_
                        g.N, g.epi, g.C, g.ldc);
   }
   return vh::check_launch("vh_gemm_nf4");
+}
+
+// ------------------------------------------------------------ MXNF4 prefill, decoded activation
+// The same product on an activation decoded once to bf16(level * scale)
+// [M, K]: its stages go straight into LDS (buffer_load_dwordx4 ... lds, rows
+// swizzled as k_gemm_f8dl's), and the weight never passes through LDS as
+// bf16: a wave decodes the GEMV records of its own columns in registers,
+// where record lane r + 16 c already is the row operand of
+// v_mfma_f32_16x16x32_bf16 (column r of the tile, elements 16 c .. + 7 in
+// the block's first MFMA and the next 8 in its second).
+//
+// Per 64-element block a wave spends about 68 VALU instructions a 16-column
+// tile on the decode and 2 TM MFMAs of 16 cycles a tile, so the row tile is
+// as tall as the accumulators allow and covers all rows up to 256: each
+// weight element is decoded WM times on the chip instead of once per row
+// tile of 128.  WM = 2 above 128 rows (both halves decode the same columns,
+// each x fragment serves two MFMAs), WM = 1 below (the decode would cost
+// more than the fragment reads).  One wave per SIMD issues about one
+// instruction in eight cycles here and leaves the decode and the MFMAs end
+// to end, so KG groups of four waves take the blocks of a stage in turn and
+// add their sums through LDS at the end.
+//
+// A stage is KG blocks.  In stage s the DMA of x stage s + NX - 1 and of the
+// records of stage s + NX + 1 goes out, the MFMAs run on the fragments
+// decoded during stage s - 1, and the records of stage s + 1 are decoded
+// between them.  A wave waits for its own DMA of x stage s + 1 and record
+// stage s + 2 and for its LDS reads before the barrier that opens stage s +
+// 1: after it both are whole and the buffers of x stage s and record stage s
+// + 1 are free.
+//
+// MI355X, us, the activation's decode not counted (k_gemm_nf4 beside it):
+// (K, N) = (4096, 14336) at 17 / 64 / 128 / 201 / 256 rows: 16.5 / 21.3 /
+// 32.2 / 49.5 / 53.7 (42.5 / 46.0 / 48.8 / 78.2 / 78.5); (14336, 4096): 16.9
+// / 22.6 / 31.4 / 47.4 / 50.7 (41.2 / 44.8 / 46.0 / 76.4 / 77.0).  At 201
+// rows the x stages alone take 35 us (every workgroup reads all of x from
+// L2), the rest without them 44, of which decode and MFMAs 10 and 12; with
+// one wave per SIMD 55.
+constexpr int NF4B_BN = 64;
+constexpr int NF4B_MAX_KCS = 256;  // blocks of a K range: its scale codes lie in LDS
+
+// The (column, block) scale codes of a range come after the rings.
+template <int BM, int KG, int NX>
+constexpr int nf4b_lds(int kcs) {
+  return KG * (NX * BM * 128 + (NX + 1) * NF4B_BN * 32) + 1040 + kcs * NF4B_BN;
+}
+
+template <int BM, int WM, int KG, int NX>
+__global__ void __launch_bounds__(KG * 256, KG) __attribute__((amdgpu_waves_per_eu(KG, KG)))
+k_gemm_nf4_bf16(GemmArgs g, Nf4Args q, int mt, int tiles, int kcs, float* __restrict__ part) {
+  constexpr int BN = NF4B_BN, WN = 4 / WM;
+  constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+  constexpr int XB = BM * 128, WB = BN * 32;  // bytes of one block of x and of records
+  constexpr int LX = BM / 32, L = LX + 1;     // DMA instructions per wave and stage
+  static_assert(BM % 32 == 0 && NX >= 2, "bad tile");
+  static_assert((KG - 1) * BM * BN * 4 <= KG * NX * XB, "the partial sums must fit the x ring");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  uint8_t* s_w = smem + KG * NX * XB;                    // [NX + 1][KG] records
+  float* s_sb = (float*)(s_w + KG * (NX + 1) * WB);      // [257] values of the scale codes, 0
+  uint8_t* s_sc = (uint8_t*)(s_sb + 260);                // [BN / 16][kcs][16] scale codes
+  // blocks go to the XCDs round-robin: an XCD takes a run of tiles, row
+  // tiles of the same columns next to each other, so their weight is read
+  // into one L2
+  const int per = (tiles + 7) / 8;
+  const int t = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (t >= tiles) return;
+  const int64_t m0 = (int64_t)(t % mt) * BM, n0 = (int64_t)(t / mt) * BN;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
+  const int kg = __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int wm = wave / WN, wn = wave % WN;
+  const int nbk = (int)(g.K / 64);
+  const int kb0 = (int)blockIdx.y * kcs;
+  const int nk = (nbk - kb0) < kcs ? (nbk - kb0) : kcs;
+  const int64_t rows_a = (g.M - m0) < BM ? (g.M - m0) : BM;
+  const int64_t rows_b = (g.N - n0) < BN ? (g.N - n0) : BN;  // a multiple of 16
+  const i32x4 ra = raw_desc(g.A + m0 * g.lda, rows_a * g.lda);
+  const i32x4 rb = raw_desc(g.B + (n0 / 16) * nbk * 512, rows_b / 16 * nbk * 512);
+  const rsrc_t bs = make_rsrc(g.b_scale + (n0 / 16) * nbk * 16, rows_b / 16 * nbk * 16);
+  uint32_t base;
+  asm volatile("v_mov_b32 %0, 0x3020100" : "=v"(base));
+  const uint32_t lds_x = (uint32_t)(uintptr_t)(lds_void*)smem + kg * XB;
+  const uint32_t lds_w = (uint32_t)(uintptr_t)(lds_void*)s_w + kg * WB;
+
+  // A wave brings in blocks of its own group.  x instruction d: rows 8 (4 d
+  // + wave) .. + 7, lane -> row lane / 8, stored chunk lane % 8; blocks past
+  // the range's end read zeros
+  const int drow = wave * 8 + (lane >> 3);
+  const int vx0 = drow * (int)g.lda + ((lane & 7) ^ swz<128>(drow & 15)) * 16 + (kb0 + kg) * 128;
+  const int vw0 = (wave * nbk + kb0 + kg) * 512 + lane * 16;
+  const int vstep = 32 * (int)g.lda;
+  auto x_in = [&](int s, int buf) {
+    const bool live = s * KG + kg < nk;
+#pragma unroll
+    for (int d = 0; d < LX; ++d)
+      dma16(ra, lds_x + buf * (KG * XB) + (4 * d + wave) * 1024,
+            live ? vx0 + d * vstep + s * (KG * 128) : (int)0x80000000);
+  };
+  auto w_in = [&](int s, int buf) {
+    const bool live = s * KG + kg < nk;
+    dma16_half(rb, lds_w + buf * (KG * WB) + wave * 512, live ? vw0 + s * (KG * 512) : (int)0x80000000);
+  };
+
+#pragma unroll
+  for (int s = 0; s < NX - 1; ++s) x_in(s, s);
+#pragma unroll
+  for (int s = 0; s < NX + 1; ++s) w_in(s, s);
+  for (int i = tid; i < 4 * kcs; i += KG * 256) {
+    const int tile = i / kcs, kb = i - tile * kcs;
+    *(uint4*)(s_sc + i * 16) = bload16(bs, (tile * nbk + kb0 + kb) * 16);
+  }
+  if (tid < 256) s_sb[tid] = fmt_decode((uint32_t)tid, q.b_sf, nullptr);
+  if (tid == 0) s_sb[256] = 0.0f;
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int l16 = lane & 15, c4 = lane >> 4;
+  const int fsw = swz<128>(l16);
+  const uint8_t* xrow = smem + kg * XB + (wm * TM * 16 + l16) * 128;
+  const uint8_t* wrec = s_w + kg * WB + wn * TN * 512 + lane * 8;
+  const uint8_t* scb = s_sc + wn * TN * kcs * 16 + l16;
+
+  // Past the range's end the scale is 0: the block's fragments are zeros
+  // (x is, too).
+  auto code = [&](int s, int j) {
+    const int b = s * KG + kg;
+    const uint32_t c = scb[(j * kcs + (b < nk ? b : nk - 1)) * 16];
+    return b < nk ? c : 256u;
+  };
+  uint2 w[TN];           // records of the stage to decode next
+  uint32_t sc_code[TN];  // scale codes of the stage after it
+  float scale[TN];       // its scales
+  uint4 wf[TN][2];       // fragments of the stage to multiply
+  // x fragment k of a stage: row tile k % TM, half k / TM of the block's MFMAs
+  auto fragment = [&](const uint8_t* xb, int k) {
+    return *(const bf16x8*)(xb + (k % TM) * 2048 + (((2 * c4 + k / TM) ^ fsw) << 4));
+  };
+  auto records = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      w[j] = *(const uint2*)(wrec + buf * (KG * WB) + j * 512);
+      scale[j] = s_sb[sc_code[j]];
+    }
+  };
+  wait_vmcnt<0>();
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < TN; ++j) sc_code[j] = code(0, j);
+  records(0);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    sc_code[j] = code(1, j);
+    const uint32_t l[4] = {lut_lo(w[j].x, base, q.lvb), lut_lo(w[j].y, base, q.lvb),
+                           lut_hi(w[j].x, base, q.lvb), lut_hi(w[j].y, base, q.lvb)};
+    nf4_pack16(l, scale[j], wf[j][0], wf[j][1]);
+  }
+  const int ns = (nk + KG - 1) / KG;
+  int xbuf = 0, wbuf = 0;
+  for (int s = 0; s < ns; ++s) {
+    wait_vmcnt<(NX - 2) * L + 1>();
+    lds_barrier();
+    x_in(s + NX - 1, xbuf == 0 ? NX - 1 : xbuf - 1);
+    w_in(s + NX + 1, wbuf);
+    wbuf = wbuf == NX ? 0 : wbuf + 1;
+    records(wbuf);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) sc_code[j] = code(s + 2, j);
+    // Groups of TN MFMAs on one x fragment, read AHEAD groups before; the
+    // decode's 8 TN steps (the levels of four elements, then their products)
+    // are spread evenly over the groups that follow the records' latency.
+    constexpr int G = 2 * TM, U = 8 * TN, LEAD = G > 4 ? 2 : 1, AHEAD = 3;
+    const uint8_t* xb = xrow + xbuf * (KG * XB);
+    bf16x8 xf[AHEAD];
+    uint32_t lv = 0;
+    uint32_t nf[TN][8];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) xf[k] = fragment(xb, k);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        acc[k % TM][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[j][k / TM]),
+                                                                 xf[k % AHEAD], acc[k % TM][j], 0, 0, 0);
+      if (k + AHEAD < G) xf[k % AHEAD] = fragment(xb, k + AHEAD);
+      if (k >= LEAD) {
+#pragma unroll
+        for (int u = (k - LEAD) * U / (G - LEAD); u < (k + 1 - LEAD) * U / (G - LEAD); ++u) {
+          const int j = u >> 3, d = (u >> 1) & 3;
+          if ((u & 1) == 0) {
+            const uint32_t r = (d & 1) ? w[j].y : w[j].x;
+            lv = d < 2 ? lut_lo(r, base, q.lvb) : lut_hi(r, base, q.lvb);
+          } else {
+            float f[4];
+            nf4_levels4(lv, scale[j], -128.0f * scale[j], f);
+            nf[j][2 * d] = f2bf2_hw(f[0], f[1]);
+            nf[j][2 * d + 1] = f2bf2_hw(f[2], f[3]);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      wf[j][0] = make_uint4(nf[j][0], nf[j][1], nf[j][2], nf[j][3]);
+      wf[j][1] = make_uint4(nf[j][4], nf[j][5], nf[j][6], nf[j][7]);
+    }
+    xbuf = xbuf == NX - 1 ? 0 : xbuf + 1;
+  }
+  wait_vmcnt<0>();
+
+  // the groups' sums: each other group's in its own part of the x ring, one
+  // float4 per lane and tile
+  if constexpr (KG > 1) {
+    lds_barrier();
+    f32x4* s_acc = (f32x4*)smem;
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          s_acc[(((kg - 1) * 4 + wave) * (TM * TN) + i * TN + j) * 64 + lane] = acc[i][j];
+    }
+    lds_barrier();
+    if (kg > 0) return;
+#pragma unroll
+    for (int o = 0; o < KG - 1; ++o)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += s_acc[((o * 4 + wave) * (TM * TN) + i * TN + j) * 64 + lane];
+  }
+
+  const float sc = part ? 1.0f : epi_scale(g.epi);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int64_t col = n0 + (wn * TN + j) * 16 + c4 * 4;
+    if (col >= g.N) continue;
+    float b[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b[r] = part ? 0.0f : epi_bias(g.epi, col + r);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int64_t row = m0 + (wm * TM + i) * 16 + l16;
+      if (row >= g.M) continue;
+      const f32x4 a = acc[i][j];
+      if (part) {
+        *(f32x4*)(part + ((int64_t)blockIdx.y * g.M + row) * g.N + col) = a;
+        continue;
+      }
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = epi_value(g.epi, a[r], sc, b[r]);
+      if (g.epi.out_dtype == VH_BF16)
+        *(uint2*)((uint16_t*)g.C + row * g.ldc + col) =
+            make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                       (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+      else
+        *(f32x4*)((float*)g.C + row * g.ldc + col) = f32x4{v[0], v[1], v[2], v[3]};
+    }
+  }
+}
+
+struct Nf4bPlan {
+  int bm, wm, mt, tiles, splits, kcs;
+};
+
+inline Nf4bPlan nf4b_plan(int64_t M, int64_t N, int64_t K, int splits) {
+  Nf4bPlan p;
+  p.mt = (int)((M + 255) / 256);
+  const int per = (int)((M + p.mt - 1) / p.mt);  // rows a tile has to cover
+  p.wm = per > 128 ? 2 : 1;
+  p.bm = (per + 31) / 32 * 32;
+  if (p.bm < 160 && p.bm > 64) p.bm = p.bm > 96 ? 128 : 96;
+  p.tiles = (int)(p.mt * ((N + NF4B_BN - 1) / NF4B_BN));
+  const int nbk = (int)(K / 64);
+  int sp = splits;
+  if (sp <= 0) {
+    sp = p.tiles >= 160 ? 1 : (256 + p.tiles / 2) / p.tiles;
+    if (sp > nbk / 4) sp = nbk / 4;
+  }
+  const int least = (nbk + NF4B_MAX_KCS - 1) / NF4B_MAX_KCS;
+  if (sp < least) sp = least;
+  if (sp > nbk) sp = nbk;
+  p.kcs = (nbk + sp - 1) / sp;
+  p.splits = (nbk + p.kcs - 1) / p.kcs;  // every range has at least one block
+  return p;
+}
+
+template <int BM, int WM, int KG, int NX>
+int launch_nf4b(const GemmArgs& g, const Nf4Args& q, const Nf4bPlan& p, float* part, hipStream_t stream) {
+  static_assert(nf4b_lds<BM, KG, NX>(NF4B_MAX_KCS) <= 160 * 1024, "LDS");
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)k_gemm_nf4_bf16<BM, WM, KG, NX>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            nf4b_lds<BM, KG, NX>(NF4B_MAX_KCS)) != hipSuccess) {
+      vh::set_error("vh_gemm_nf4_bf16: cannot reserve %d bytes of LDS", nf4b_lds<BM, KG, NX>(NF4B_MAX_KCS));
+      return VH_ELAUNCH;
+    }
+    attr_set = true;
+  }
+  const size_t lds = nf4b_lds<BM, KG, NX>(p.kcs);
+  hipLaunchKernelGGL((k_gemm_nf4_bf16<BM, WM, KG, NX>), dim3((unsigned)((p.tiles + 7) / 8 * 8), (unsigned)p.splits),
+                     dim3(KG * 256), lds, stream, g, q, p.mt, p.tiles, p.kcs,
+                     p.splits > 1 ? part : nullptr);
+  if (p.splits > 1) {
+    const int64_t quads = g.M * g.N / 4;
+    hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, part, p.splits,
+                       g.M, g.N, g.epi, g.C, g.ldc);
+  }
+  return vh::check_launch("vh_gemm_nf4_bf16");
 }
 
 // ------------------------------------------------------------ MXNF4 operands to bf16
@@ -2536,6 +2835,72 @@ extern "C" int vh_gemm_nf4_plan(int64_t M, int64_t N, int64_t K, int32_t* tile, 
   const int64_t nbk = K / 64, kcs = (nbk + *splits - 1) / *splits;
   *splits = (int32_t)((nbk + kcs - 1) / kcs);
   return VH_OK;
+}
+
+extern "C" int vh_gemm_nf4_bf16_plan(int64_t M, int64_t N, int64_t K, int32_t* splits) {
+  VH_REQUIRE(splits && M >= 1 && N > 0 && K >= 64, "vh_gemm_nf4_bf16_plan: bad arguments");
+  *splits = nf4b_plan(M, N, K, *splits).splits;
+  return VH_OK;
+}
+
+extern "C" int vh_gemm_nf4_bf16(const uint16_t* x, int64_t M, const uint8_t* w_packed, const uint8_t* w_scale,
+                                const vh_format* w_scale_fmt, const int8_t* levels16, int64_t N, int64_t K,
+                                const vh_epilogue* epi, void* y, int64_t ldy, int32_t splits, float* part,
+                                int64_t part_bytes, vh_stream_t stream) {
+  VH_REQUIRE(x && w_packed && w_scale && w_scale_fmt && levels16 && epi && y, "vh_gemm_nf4_bf16: null argument");
+  VH_REQUIRE(M >= 1 && N > 0 && K > 0 && N % 16 == 0 && K % 64 == 0,
+             "vh_gemm_nf4_bf16: needs N %% 16 == 0 and K %% 64 == 0");
+  VH_REQUIRE((N / 16) * (K / 64) * 512 < (1ll << 31), "vh_gemm_nf4_bf16: operands over 2 GiB");
+  // a workgroup's offsets (at most 256 rows, 64 columns) are 32 bits
+  VH_REQUIRE(K <= (1 << 20) && M < (1ll << 24) && N < (1ll << 24), "vh_gemm_nf4_bf16: operands too large");
+  VH_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)w_packed % 16 == 0 && (uintptr_t)w_scale % 16 == 0 &&
+                 (uintptr_t)y % 16 == 0 && (uintptr_t)part % 16 == 0,
+             "vh_gemm_nf4_bf16: misaligned operand");
+  VH_REQUIRE(epi->mode == EPI_PLAIN && (epi->out_dtype == VH_BF16 || epi->out_dtype == VH_F32) && ldy >= N &&
+                 ldy % 4 == 0,
+             "vh_gemm_nf4_bf16: unsupported epilogue");
+  VH_REQUIRE(!epi->scale || epi->scale_dtype == VH_BF16 || epi->scale_dtype == VH_F32,
+             "vh_gemm_nf4_bf16: scale must be bf16 or float32");
+  VH_REQUIRE(!epi->bias || epi->bias_dtype == VH_BF16 || epi->bias_dtype == VH_F32,
+             "vh_gemm_nf4_bf16: bias must be bf16 or float32");
+  VH_REQUIRE(w_scale_fmt->kind == VH_FMT_INT || w_scale_fmt->kind == VH_FMT_MINIFLOAT ||
+                 w_scale_fmt->kind == VH_FMT_POSIT,
+             "vh_gemm_nf4_bf16: the scale map needs a closed form with packed codes");
+  const Nf4bPlan p = nf4b_plan(M, N, K, splits);
+  VH_REQUIRE(p.splits == 1 || (part && part_bytes >= (int64_t)p.splits * M * N * 4 && ldy == N),
+             "vh_gemm_nf4_bf16: %d K splits need a workspace of %lld bytes (and ldy == N)", p.splits,
+             (long long)((int64_t)p.splits * M * N * 4));
+  Nf4Args q;
+  memset(&q, 0, sizeof(q));
+  uint8_t lvb[16];
+  for (int v = 0; v < 16; ++v) lvb[v] = (uint8_t)(levels16[v] + 128);
+  uint32_t t[4];
+  memcpy(t, lvb, 16);
+  q.lvb = make_uint4(t[0], t[1], t[2], t[3]);
+  q.b_sf = *w_scale_fmt;
+  GemmArgs g;
+  memset(&g, 0, sizeof(g));
+  g.A = (const uint8_t*)x;
+  g.B = w_packed;
+  g.C = y;
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.lda = K * 2;
+  g.ldc = ldy;
+  g.b_scale = w_scale;
+  g.epi = *epi;
+  hipStream_t st = vh::as_stream(stream);
+  switch (p.bm) {
+    case 32: return launch_nf4b<32, 1, 4, 3>(g, q, p, part, st);
+    case 64: return launch_nf4b<64, 1, 4, 3>(g, q, p, part, st);
+    case 96: return launch_nf4b<96, 1, 2, 3>(g, q, p, part, st);
+    case 128: return launch_nf4b<128, 1, 2, 3>(g, q, p, part, st);
+    case 160: return launch_nf4b<160, 2, 2, 2>(g, q, p, part, st);
+    case 192: return launch_nf4b<192, 2, 2, 2>(g, q, p, part, st);
+    case 224: return launch_nf4b<224, 2, 2, 2>(g, q, p, part, st);
+    default: return launch_nf4b<256, 2, 2, 2>(g, q, p, part, st);
+  }
 }
 
 extern "C" int vh_nf4_decode_bf16(const uint8_t* x_idx, const uint8_t* x_scale, const vh_format* x_scale_fmt,

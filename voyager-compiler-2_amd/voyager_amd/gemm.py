@@ -624,9 +624,16 @@ def _level_lut(levels: bytes, device) -> torch.Tensor:
 def _nf4_fusable(x: torch.Tensor, ec, sc) -> bool:
     """Whether ``vh_gemv_nf4_m1`` can take this call: one bfloat16 row, a
     minifloat activation scale map and an index table of at most 16 levels."""
+    return x.shape[0] == 1 and _nf4_index_quantize(x, ec, sc)
+
+
+def _nf4_index_quantize(x: torch.Tensor, ec, sc) -> bool:
+    """Bfloat16 rows under a minifloat scale map and an index table of at
+    most 16 levels: what the kernels that quantize MXNF4 activations without
+    writing their codes take."""
     f, s = ec.fmt, sc.fmt
-    return (x.shape[0] == 1 and x.dtype == torch.bfloat16 and s.kind == FMT_MINIFLOAT
-            and not (s.flags & FMT_HW_E4M3) and f.kind == FMT_STEPS and f.nsteps <= 15 and f.nan_level <= 15)
+    return (x.dtype == torch.bfloat16 and s.kind == FMT_MINIFLOAT and not (s.flags & FMT_HW_E4M3)
+            and f.kind == FMT_STEPS and f.nsteps <= 15 and f.nan_level <= 15)
 
 
 def _nf4_one_launch_pays(N: int, K: int) -> bool:
@@ -648,18 +655,44 @@ def nf4_prefill_plan(M: int, N: int, K: int, tile: int = 0, splits: int = 0) -> 
 def linear_nf4_prefill(x: torch.Tensor, weight: NF4Weight, index_table: torch.Tensor, scale_qmap: torch.Tensor,
                        out_dtype=torch.bfloat16, bias=None, alpha=None, tile: int = 0,
                        splits: int = 0, two_pass: Optional[bool] = None) -> torch.Tensor:
-    """MXNF4 ``linear_mx`` at any M on the GEMV's baked weight: the
-    activation's ``quantize_mx`` to index and scale bytes, then
-    ``vh_gemm_nf4``, which decodes both operands while staging to the
-    reference's ``bf16(level * scale)`` and multiplies them on the bf16 MFMA
-    with float32 accumulation."""
+    """MXNF4 ``linear_mx`` at any M on the GEMV's baked weight: both operands
+    decoded to the reference's ``bf16(level * scale)`` and multiplied on the
+    bf16 MFMA with float32 accumulation.  Up to 256 rows (and by few columns,
+    ``nf4_two_pass_pays``) the activation is quantized straight to those
+    values and the weight decoded in the GEMM (``vh_gemm_nf4_bf16``); else,
+    or at a given ``tile`` / ``splits`` / ``two_pass``, its ``quantize_mx``
+    goes to index and scale bytes for ``gemm_nf4_packed``."""
     from . import packed as _packed
 
     M, K = x.shape
     if K != weight.K:
         raise RuntimeError("linear_nf4_prefill: contraction mismatch")
-    px = _packed.quantize_mx_packed(x.contiguous(), index_table, [-1], 64, 31.0, False, scale_qmap)
+    x = x.contiguous()
+    if two_pass is None and tile == 0 and splits == 0 and _nf4_bf16_pays(M, weight):
+        ec, sc = formats.classify(index_table), formats.classify(scale_qmap)
+        if _nf4_index_quantize(x, ec, sc) and x.data_ptr() % 16 == 0:
+            return gemm_nf4_bf16(nf4_quantize_bf16(x, weight, ec, sc), weight, out_dtype, bias, alpha)
+    px = _packed.quantize_mx_packed(x, index_table, [-1], 64, 31.0, False, scale_qmap)
     return gemm_nf4_packed(px, weight, out_dtype, bias, alpha, tile, splits, two_pass)
+
+
+def _nf4_bf16_pays(M: int, weight: NF4Weight) -> bool:
+    """Whether ``vh_gemm_nf4_bf16`` takes the prefill: where
+    ``nf4_two_pass_pays`` does not, and the weight lies as its loads need."""
+    return (M >= 1 and not nf4_two_pass_pays(M, weight.N, weight.K) and weight.K <= 1 << 20
+            and weight.packed.data_ptr() % 16 == 0 and weight.scale.data_ptr() % 16 == 0)
+
+
+def nf4_quantize_bf16(x: torch.Tensor, weight: NF4Weight, ec, sc) -> torch.Tensor:
+    """``vh_nf4_quantize_bf16``: the MXNF4 ``quantize_mx`` of x [M, K] as the
+    bf16 values its codes decode to (``quantize_mx_packed`` then
+    ``nf4_decode_bf16``, in one pass)."""
+    out = torch.empty_like(x)
+    lv = ctypes.create_string_buffer(weight.levels, 16)
+    st = load().vh_nf4_quantize_bf16(ptr(x), x.shape[0], x.shape[1], 31.0, ctypes.byref(sc.fmt), ctypes.byref(ec.fmt),
+                                     lv, ptr(out), ctypes.c_void_p(stream_of(x)))
+    _lib.check(st, "vh_nf4_quantize_bf16")
+    return out
 
 
 def nf4_decode_bf16(px, weight: NF4Weight, decode_x: bool = True, decode_w: bool = True):
@@ -685,32 +718,41 @@ def nf4_decode_bf16(px, weight: NF4Weight, decode_x: bool = True, decode_w: bool
 
 def nf4_two_pass_pays(M: int, N: int, K: int) -> bool:
     """Whether the prefill runs as two passes (both operands decoded once,
-    then the bf16 GEMM) rather than ``vh_gemm_nf4``, which decodes each
-    weight block once per row tile of the output.  Measured on MI355X
-    (fused / two-pass, us): (K, N) = (4096, 4096) at M = 256: 35.1 / 37.5,
-    M = 512: 49.8 / 37.4, M = 2048: 96.3 / 74.4; (4096, 14336): 78.0 / 57.8,
-    95.4 / 79.5, 368.7 / 227.9; (14336, 4096): 77.1 / 90.1, 140.8 / 98.7,
-    321.1 / 219.1.  The two-pass form holds the decoded weight (2 bytes per
-    element) for the call."""
-    return M >= NF4_TWO_PASS_MIN_M
+    then the bf16 GEMM) rather than on ``vh_gemm_nf4_bf16``, which decodes a
+    weight block once per 256 rows and multiplies at half the bf16 GEMM's
+    rate.  Measured on MI355X (``vh_gemm_nf4_bf16`` with the activation's
+    decode / two-pass, us): (K, N) = (4096, 4096) at M = 256: 29.6 / 32.5,
+    300: 32.0 / 32.7, 512: 39.1 / 34.2; (4096, 14336): 57.5 / 58.9, 84.2 /
+    72.1, 103 / 77.9; (14336, 4096): 55.5 / 87.3, 73.5 / 94.7, 99.9 / 102;
+    (4096, 1024): 25.8 / 26.8, 21.8 / 30.5, 24.5 / 30.5.  So up to 256 rows
+    the one tile of rows decides, and above them only columns too few to
+    fill the chip do.  The two-pass form holds the decoded weight (2 bytes
+    per element) for the call."""
+    return M >= NF4_TWO_PASS_MIN_M or (M > 256 and N > 2048)
 
 
-#: Rows from which the two-pass MXNF4 prefill is taken.
+#: Rows from which the two-pass MXNF4 prefill is taken at every N.
 NF4_TWO_PASS_MIN_M = 512
 
 
 def gemm_nf4_packed(px, weight: NF4Weight, out_dtype=torch.bfloat16, bias=None, alpha=None, tile: int = 0,
                     splits: int = 0, two_pass: Optional[bool] = None) -> torch.Tensor:
-    """``vh_gemm_nf4`` on an activation already packed by ``quantize_mx_packed``
-    (index bytes [M, K] and scale codes [M, K / 64]); with ``two_pass`` (by
-    default where ``nf4_two_pass_pays``) the operands decoded once by
-    ``nf4_decode_bf16`` and multiplied by the bf16 GEMM instead, which gives
-    the same products summed in another order."""
+    """The MXNF4 linear of an activation already packed by
+    ``quantize_mx_packed`` (index bytes [M, K] and scale codes [M, K / 64]):
+    with ``two_pass`` (by default where ``nf4_two_pass_pays``) the operands
+    decoded once by ``nf4_decode_bf16`` and multiplied by the bf16 GEMM;
+    without, or at a given tile or split, ``vh_gemm_nf4``, which decodes both
+    while staging; by default below that the activation decoded once and
+    ``vh_gemm_nf4_bf16``.  All give the same products, summed in another
+    order."""
     M, K = px.codes.shape
     if K != weight.K:
         raise RuntimeError("gemm_nf4_packed: contraction mismatch")
     if two_pass is None:
         two_pass = nf4_two_pass_pays(M, weight.N, K)
+        if tile == 0 and splits == 0 and _nf4_bf16_pays(M, weight):
+            xo, _ = nf4_decode_bf16(px, weight, decode_w=False)
+            return gemm_nf4_bf16(xo, weight, out_dtype, bias, alpha)
     if two_pass:
         xo, wo = nf4_decode_bf16(px, weight)
         return gemm_bf16(xo, wo, out_dtype, bias, alpha)
@@ -729,6 +771,32 @@ def gemm_nf4_packed(px, weight: NF4Weight, out_dtype=torch.bfloat16, bias=None, 
                             ctypes.c_void_p(y.data_ptr()), weight.N, tile, splits, ptr(part),
                             0 if part is None else part.numel() * 4, ctypes.c_void_p(stream_of(y)))
     _lib.check(st, "vh_gemm_nf4")
+    return y
+
+
+def gemm_nf4_bf16(x: torch.Tensor, weight: NF4Weight, out_dtype=torch.bfloat16, bias=None, alpha=None,
+                  splits: int = 0) -> torch.Tensor:
+    """``vh_gemm_nf4_bf16``: the MXNF4 linear of an activation already decoded
+    to bfloat16 [M, K] (``nf4_decode_bf16``), the weight decoded in the
+    GEMM's registers."""
+    M, K = x.shape
+    if K != weight.K or x.dtype != torch.bfloat16 or not x.is_contiguous():
+        raise RuntimeError("gemm_nf4_bf16: contraction mismatch")
+    y = torch.empty(M, weight.N, dtype=out_dtype, device=x.device)
+    if alpha is not None:
+        alpha = alpha.reshape(()).to(torch.float32).contiguous()
+    bias = _bias_operand(bias)
+    epi = _epilogue(EPI_PLAIN, out_dtype, alpha, bias)
+    lv = ctypes.create_string_buffer(weight.levels, 16)
+    sp = ctypes.c_int32(splits)
+    _lib.check(load().vh_gemm_nf4_bf16_plan(M, weight.N, K, ctypes.byref(sp)), "vh_gemm_nf4_bf16_plan")
+    part = torch.empty(sp.value * M * weight.N, dtype=torch.float32, device=y.device) if sp.value > 1 else None
+    st = load().vh_gemm_nf4_bf16(ctypes.c_void_p(x.data_ptr()), M, ctypes.c_void_p(weight.packed.data_ptr()),
+                                 ctypes.c_void_p(weight.scale.data_ptr()), ctypes.byref(weight.scale_fmt.fmt), lv,
+                                 weight.N, K, ctypes.c_void_p(ctypes.addressof(epi)),
+                                 ctypes.c_void_p(y.data_ptr()), weight.N, sp.value, ptr(part),
+                                 0 if part is None else part.numel() * 4, ctypes.c_void_p(stream_of(y)))
+    _lib.check(st, "vh_gemm_nf4_bf16")
     return y
 
 
