@@ -294,8 +294,8 @@ int64_t vh_gemm_workspace_bytes(const vh_gemm_desc* desc);
 /* The kernel vh_gemm runs for `desc` (the same rule, evaluated on the host;
  * the output pointer C enters through its alignment): family 1 the
  * register-staged kernel (tiles 2..10 as tile_hint names them), 2 the
- * direct-to-LDS kernel on E4M3 operands (tiles 20..43), 3 the direct-to-LDS
- * kernel on bf16 operands (31, 33, 35, 37, 41), 4 the MX-int8 kernels
+ * direct-to-LDS kernel on E4M3 operands (tiles 20..48), 3 the direct-to-LDS
+ * kernel on bf16 operands (25, 26, 31, 33, 35, 37, 41), 4 the MX-int8 kernels
  * (50..56) with `splits` K splits.  No counterpart in the reference, whose
  * GEMM is one aten call; tests use it to assert which tile a shape takes. */
 #define VH_GEMM_FAMILY_STAGED 1
@@ -330,10 +330,14 @@ int vh_gemm_plan(const vh_gemm_desc* desc, int32_t* family, int32_t* tile, int32
  * multiples of 8 for bf16, ldy of 4 for float32) the GEMM applies the
  * exponents and the epilogue itself and `part` may be null; tile 0:
  * 128x128, 1: 64x128, 2: 128x64, 3: 256x128, 4: 64x64 (two waves, eight
- * stages in flight: the small-M tile).  No
+ * stages in flight: the small-M tile), 5: 128x192, 6: 256x160, 7: 256x256.  No
  * reference counterpart for the operand form: it is this library's
  * small-M layout of the same values. */
 int vh_quantize_mx8_f16(const uint16_t* x, int64_t M, int64_t K, uint16_t* out, int32_t* ex, vh_stream_t stream);
+/* The same with a NaN element as the code 0 that vh_quantize_mx packs for
+ * it: the rows vh_mx8_bake_f16 makes of the packed codes, in one pass. */
+int vh_quantize_mx8_f16_codes(const uint16_t* x, int64_t M, int64_t K, uint16_t* out, int32_t* ex,
+                              vh_stream_t stream);
 int vh_mx8_bake_f16(const int8_t* codes, const uint8_t* scale, int32_t scale_bias, int64_t N, int64_t K,
                     uint16_t* out, int32_t* ew, vh_stream_t stream);
 int vh_gemm_mx8_f16(const uint16_t* x, const int32_t* ex, const uint16_t* w, const int32_t* ew, int64_t M,

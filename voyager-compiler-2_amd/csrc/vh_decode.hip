@@ -204,6 +204,7 @@ VH_DEV int block_max_int(int v, int* s_red) {
 // bf16 row (ops/quantized.py:1070-1115; codes and scales as mx8_scale /
 // mx8_fq form them), written as the exact fp16 row above with E in ex.  One
 // workgroup per row: the blocks' exponents, their maximum, then the codes.
+template <bool CODES>
 __global__ void __launch_bounds__(256) k_quantize_mx8_f16(const uint16_t* __restrict__ x, int64_t K,
                                                           _Float16* __restrict__ out, int32_t* __restrict__ ex) {
   __shared__ int s_red[4];
@@ -241,6 +242,7 @@ __global__ void __launch_bounds__(256) k_quantize_mx8_f16(const uint16_t* __rest
     for (int j = 0; j < 16; ++j) {
       float q = rbf(sc.pow2 ? ldexpf(xv[j], -sc.e) : xv[j] / sc.s);
       if (!isnan_f(q)) q = fminf(fmaxf(rintf(q), -128.0f), 127.0f);
+      else if (CODES) q = 0.0f;
       o[j >> 3][j & 7] = rebased_f16(q, sc.e, sc.pow2, sc.s, E);
     }
     f16x8* dst = (f16x8*)(out + row * K + b * 16);
@@ -252,8 +254,9 @@ __global__ void __launch_bounds__(256) k_quantize_mx8_f16(const uint16_t* __rest
 
 // The same for rows of at most 256 NBT blocks: each thread loads its NBT
 // blocks once and keeps them in registers across the row maximum (no second
-// read of the row); identical arithmetic, so identical output.
-template <int NBT>
+// read of the row); identical arithmetic, so identical output.  CODES: a NaN
+// element is the code 0 that the packed codes hold for it.
+template <int NBT, bool CODES>
 __global__ void __launch_bounds__(256) k_quantize_mx8_f16_r(const uint16_t* __restrict__ x, int64_t K,
                                                             _Float16* __restrict__ out, int32_t* __restrict__ ex) {
   __shared__ int s_red[4];
@@ -302,7 +305,7 @@ __global__ void __launch_bounds__(256) k_quantize_mx8_f16_r(const uint16_t* __re
     for (int i = 0; i < 16; ++i) {
       const float xv = bf2f((i & 1) ? wv[i >> 1] >> 16 : wv[i >> 1] & 0xffffu);
       float q = rbf(p2 ? ldexpf(xv, -sc[j].e) : xv * 0.0f);
-      q = isnan_f(q) ? q : fminf(fmaxf(rintf(q), -128.0f), 127.0f);
+      q = isnan_f(q) ? (CODES ? 0.0f : q) : fminf(fmaxf(rintf(q), -128.0f), 127.0f);
       o[i >> 3][i & 7] = (_Float16)(p2 ? (keep ? ldexpf(q, d) : q * 0.0f) : q * sc[j].s);
     }
     f16x8* dst = (f16x8*)(out + row * K + (int64_t)b * 16);
@@ -1619,20 +1622,35 @@ extern "C" int vh_kivi_attention(const vh_kivi_desc* d, vh_stream_t stream) {
 
 
 
+namespace {
+template <bool CODES>
+int quantize_mx8_f16(const uint16_t* x, int64_t M, int64_t K, uint16_t* out, int32_t* ex, hipStream_t s,
+                     const char* what) {
+  VH_REQUIRE(x && out && ex, "%s: null argument", what);
+  VH_REQUIRE(M > 0 && K > 0 && K % 16 == 0, "%s: needs K a multiple of 16", what);
+  VH_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0, "%s: misaligned tensor", what);
+  const int64_t nb = K / 16;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)M), dim3(256), 0, s, x, K, (_Float16*)out, ex);
+  };
+  // up to 1024 blocks in registers (M = 1111 / 2048, K = 14336: 22.8 / 30.9
+  // us; 26.6 / 36.7 with a second read of each row)
+  if (nb <= 256) go(k_quantize_mx8_f16_r<1, CODES>);
+  else if (nb <= 512) go(k_quantize_mx8_f16_r<2, CODES>);
+  else if (nb <= 1024) go(k_quantize_mx8_f16_r<4, CODES>);
+  else go(k_quantize_mx8_f16<CODES>);
+  return vh::check_launch(what);
+}
+}  // namespace
+
 extern "C" int vh_quantize_mx8_f16(const uint16_t* x, int64_t M, int64_t K, uint16_t* out, int32_t* ex,
                                    vh_stream_t stream) {
-  VH_REQUIRE(x && out && ex, "vh_quantize_mx8_f16: null argument");
-  VH_REQUIRE(M > 0 && K > 0 && K % 16 == 0, "vh_quantize_mx8_f16: needs K a multiple of 16");
-  VH_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0, "vh_quantize_mx8_f16: misaligned tensor");
-  const int64_t nb = K / 16;
-  hipStream_t s = vh::as_stream(stream);
-  if (nb <= 256)
-    hipLaunchKernelGGL(k_quantize_mx8_f16_r<1>, dim3((unsigned)M), dim3(256), 0, s, x, K, (_Float16*)out, ex);
-  else if (nb <= 512)
-    hipLaunchKernelGGL(k_quantize_mx8_f16_r<2>, dim3((unsigned)M), dim3(256), 0, s, x, K, (_Float16*)out, ex);
-  else
-    hipLaunchKernelGGL(k_quantize_mx8_f16, dim3((unsigned)M), dim3(256), 0, s, x, K, (_Float16*)out, ex);
-  return vh::check_launch("vh_quantize_mx8_f16");
+  return quantize_mx8_f16<false>(x, M, K, out, ex, vh::as_stream(stream), "vh_quantize_mx8_f16");
+}
+
+extern "C" int vh_quantize_mx8_f16_codes(const uint16_t* x, int64_t M, int64_t K, uint16_t* out, int32_t* ex,
+                                         vh_stream_t stream) {
+  return quantize_mx8_f16<true>(x, M, K, out, ex, vh::as_stream(stream), "vh_quantize_mx8_f16_codes");
 }
 
 extern "C" int vh_mx8_bake_f16(const int8_t* codes, const uint8_t* scale, int32_t scale_bias, int64_t N, int64_t K,

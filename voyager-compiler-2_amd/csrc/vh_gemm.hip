@@ -430,16 +430,19 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, f32x16 (&acc)[TM][
 }
 
 // Block tile id -> (m0, n0).  Blocks are dealt to the 8 XCDs round robin;
-// when the tile count is a multiple of 8, consecutive tile ids are
-// renumbered so that each XCD gets a contiguous range of them, and groups of
-// GM tile-rows are walked column by column so an XCD's blocks share operand
-// panels in its L2 (group_rows picks GM).
+// tile ids are renumbered so that each XCD gets a contiguous range of them
+// (the first ntiles % 8 XCDs one more), and groups of GM tile-rows are
+// walked column by column so an XCD's blocks share operand panels in its L2
+// (group_rows picks GM).  Without the renumbering, as counts that are no
+// multiple of 8 ran before, 225 tiles of 128 x 192 (bf16, M = 300, K = 4096,
+// N = 14336) take 56.7 us against 44.0.
 __device__ __forceinline__ void tile_origin(int64_t M, int64_t N, int BM, int BN, int GM, int64_t& m0, int64_t& n0) {
   const int64_t tiles_m = (M + BM - 1) / BM;
   const int64_t tiles_n = (N + BN - 1) / BN;
   const int64_t ntiles = tiles_m * tiles_n;
   int64_t pid = blockIdx.x;
-  if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
+  const int64_t xcd = pid & 7, rest = ntiles & 7;
+  pid = xcd * (ntiles >> 3) + (xcd < rest ? xcd : rest) + (pid >> 3);
   const int64_t group = pid / (GM * tiles_n);
   const int64_t first_m = group * GM;
   const int64_t gsize = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
@@ -2464,18 +2467,57 @@ bool is_direct_fp8_tile(int c) {
   switch (c) {
     case 20: case 21: case 23: case 24: case 30: case 31: case 32: case 33: case 34:
     case 35: case 36: case 37: case 40: case 41: case 42: case 43: case 44: case 45: case 46: case 47:
-    case 48: return true;
+    case 48: case 25: case 26: return true;
     default: return false;
   }
 }
 
-bool is_direct_bf16_tile(int c) { return c == 31 || c == 33 || c == 35 || c == 37 || c == 41; }
+bool is_direct_bf16_tile(int c) {
+  return c == 31 || c == 33 || c == 35 || c == 37 || c == 41 || c == 25 || c == 26;
+}
 
 int staged_tile(int c) {
   switch (c) {
     case 2: case 3: case 5: case 6: case 7: case 8: case 9: case 10: return c;
     default: return 4;
   }
+}
+
+// Tile of a direct-to-LDS GEMM.  A CU runs one workgroup of these at a time,
+// so T tiles take ceil(T / 256) rounds of one tile's own time (c0: its MFMAs
+// and fill) plus what the running tiles cost each other in L2, HBM and clock
+// (c1 a full round's worth); the tile of the least sum is taken.  c0 and c1
+// are least-squares fits in us at K = 4096 (K scales both alike) over M =
+// 201 .. 2048 on MI355X at (K, N) = (4096, 4096), (4096, 14336), (14336,
+// 4096), every tile timed at every size; over those 36 sizes the choice is
+// within 4% of the best tile.  A choice by thresholds on the tile count
+// alone left rounds nearly empty: fp8 at M = 513 / 1111 / 1300, K = N = 4096
+// 24.6 / 32.2 / 33.3 us against 17.4 / 23.8 / 25.9 (bf16 39.1 / 54.7 / 55.4
+// against 27.2 / 40.4 / 45.3); (4096, 14336) at M = 513 / 1111 / 2048 52.9 /
+// 82.6 / 106.8 against 43.7 / 68.7 / 106.6 (bf16, M = 513 / 1111, 94.8 / 150
+// against 76.5 / 128).
+struct DlTile {
+  int tile, bm, bn;
+  float c0, c1;
+};
+constexpr DlTile DL_FP8[] = {{37, 64, 128, 10.0f, 1.8f},   {33, 128, 128, 12.4f, 5.0f},
+                             {25, 128, 192, 15.8f, 8.1f},  {31, 256, 128, 18.8f, 10.8f},
+                             {26, 256, 160, 23.2f, 12.6f}, {44, 256, 224, 41.0f, 11.2f},
+                             {41, 256, 256, 42.1f, 15.6f}};
+constexpr DlTile DL_BF16[] = {{35, 128, 64, 17.2f, 3.4f},   {33, 128, 128, 21.2f, 10.3f},
+                              {25, 128, 192, 27.8f, 15.9f}, {31, 256, 128, 33.1f, 21.6f},
+                              {26, 256, 160, 40.0f, 24.6f}, {41, 256, 256, 85.0f, 23.2f}};
+
+template <int NT>
+int dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t batch) {
+  int best = t[0].tile;
+  float least = 0.0f;
+  for (int i = 0; i < NT; ++i) {
+    const int64_t n = ((M + t[i].bm - 1) / t[i].bm) * ((N + t[i].bn - 1) / t[i].bn) * batch;
+    const float us = (float)((n + 255) / 256) * t[i].c0 + (float)n / 256.0f * t[i].c1;
+    if (i == 0 || us < least) best = t[i].tile, least = us;
+  }
+  return best;
 }
 
 // The one dispatch rule of vh_gemm: which kernel and tile a descriptor runs
@@ -2507,31 +2549,17 @@ Plan plan_gemm(const vh_gemm_desc* d) {
   // validated a multiple of 16 below, where the descriptor is checked).
   const bool chunks_ok = d->lda % 16 == 0 && d->ldb % 16 == 0 && d->K % (fp8 ? 16 : 8) == 0;
   if (fp8 && dl_ok && chunks_ok) {
-    // Direct-to-LDS kernels with 128-byte stages.  Measured on MI355X at
-    // M = 2048 (K in {4096, 14336}, N in {1024, 4096, 14336}): the largest
-    // tile that still gives every CU a block wins, since each CU's operand
-    // stream from L2 is the limit; 256 x 256 only pays when the grid covers
-    // the GPU well over once; a grid too small even for 128 x 128 takes
-    // 64 x 128 (1 x 4 waves).
-    // Where 256 x 224 tiles make whole rounds of the 256 CUs and 256 x 256
-    // tiles do not (N = 14336 = 64 x 224 at M = 2048: 512 tiles against 448,
-    // whose last round is a quarter idle), take 256 x 224 (M = 2048, K =
-    // 4096, N = 14336 under sustained load: 106.7 us against 108.7).
-    int c = d->tile_hint;
-    if (c == 0 && d->N % 224 == 0 && tiles(256, 224) >= 512 && tiles(256, 224) % 256 == 0 &&
-        tiles(256, 256) % 256 != 0)
-      c = 44;
-    if (c == 0) c = tiles(256, 256) >= 384 ? 41 : tiles(256, 128) >= 224 ? 31 : tiles(128, 128) >= 224 ? 33 : 37;
+    const int c = d->tile_hint ? d->tile_hint : dl_tile(DL_FP8, d->M, d->N, batch);
     if (is_direct_fp8_tile(c)) return {FAM_DIRECT_FP8, c, 1};
   }
   if (fp8) return {FAM_STAGED, staged, 1};
   if (d->a_fmt == OP_BF16 && d->b_fmt == OP_BF16 && dl_ok && chunks_ok && (d->tile_hint == 0 || d->tile_hint >= 20)) {
-    // As for fp8; a grid under 224 tiles of 128 x 128 takes 128 x 64
-    // (M = 256, K = 4096 on MI355X: N = 4096 in 18.5 us against 24.6 us,
-    // 21.4 against 30.1 with a float32 result; N = 14336, 224 tiles, stays
-    // at 128 x 128: 33.7 us against 46.1).
-    int c = d->tile_hint;
-    if (c == 0) c = tiles(256, 256) >= 384 ? 41 : tiles(256, 128) >= 224 ? 31 : tiles(128, 128) >= 224 ? 33 : 35;
+    // From 384 tiles of 256 x 256 those stay: the estimate would take 256 x
+    // 160 there, 192-200 us against 204-214 at M = 1800-2048, K = 4096, N =
+    // 14336 alone, but even within a run of other kernels.
+    const int c = d->tile_hint ? d->tile_hint
+                  : tiles(256, 256) >= 384 ? 41
+                                           : dl_tile(DL_BF16, d->M, d->N, batch);
     if (is_direct_bf16_tile(c)) return {FAM_DIRECT_BF16, c, 1};
   }
   if (d->a_fmt == OP_MXI8 && d->b_fmt == OP_MXI8) {
@@ -2645,6 +2673,8 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
       case 35: return launch_f8dl<128, 64, 4, 128, 2, 2>(g, batch, st);
       case 36: return launch_f8dl<128, 64, 6, 128, 2, 2>(g, batch, st);
       case 37: return launch_f8dl<64, 128, 4, 128, 1, 4>(g, batch, st);
+      case 25: return launch_f8dl<128, 192, 3, 128, 2, 2>(g, batch, st);
+      case 26: return launch_f8dl<256, 160, 3, 128, 4, 1>(g, batch, st);
       default: break;
     }
   } else if (p.family == FAM_DIRECT_BF16) {
@@ -2654,6 +2684,8 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
       case 33: return launch_f8dl<128, 128, 4, 128, 2, 2, OP_BF16>(g, batch, st);
       case 35: return launch_f8dl<128, 64, 4, 128, 2, 2, OP_BF16>(g, batch, st);
       case 37: return launch_f8dl<64, 128, 4, 128, 1, 4, OP_BF16>(g, batch, st);
+      case 25: return launch_f8dl<128, 192, 3, 128, 2, 2, OP_BF16>(g, batch, st);
+      case 26: return launch_f8dl<256, 160, 3, 128, 4, 1, OP_BF16>(g, batch, st);
       default: break;
     }
   } else if (p.family == FAM_MXI8) {
@@ -2762,6 +2794,9 @@ extern "C" int vh_gemm_mx8_f16(const uint16_t* x, const int32_t* ex, const uint1
     case 2: rc = launch_f8dl<128, 64, 4, 128, 2, 2, OP_F16X>(g, splits, st); break;
     case 3: rc = launch_f8dl<256, 128, 3, 128, 2, 2, OP_F16X>(g, splits, st); break;
     case 4: rc = launch_f8dl<64, 64, 8, 128, 1, 2, OP_F16X>(g, splits, st); break;
+    case 5: rc = launch_f8dl<128, 192, 3, 128, 2, 2, OP_F16X>(g, splits, st); break;
+    case 6: rc = launch_f8dl<256, 160, 3, 128, 4, 1, OP_F16X>(g, splits, st); break;
+    case 7: rc = launch_f8dl<256, 256, 2, 128, 4, 2, OP_F16X>(g, splits, st); break;
     default: rc = launch_f8dl<128, 128, 4, 128, 2, 2, OP_F16X>(g, splits, st); break;
   }
   if (rc || direct) return rc;

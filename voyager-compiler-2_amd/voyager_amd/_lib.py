@@ -116,6 +116,7 @@ _SIGNATURES = {
     ),
     "vh_block_amax": ([_P, _I32, _I64, _I64, _I64, _I64, _P, _P], _I32),
     "vh_quantize_mx8_f16": ([_P, _I64, _I64, _P, _P, _P], _I32),
+    "vh_quantize_mx8_f16_codes": ([_P, _I64, _I64, _P, _P, _P], _I32),
     "vh_mx8_bake_f16": ([_P, _P, _I32, _I64, _I64, _P, _P, _P], _I32),
     "vh_gemm_mx8_f16": ([_P, _P, _P, _P, _I64, _I64, _I64, _P, _P, _I64, _P, _I64, _I32, _I32, _P], _I32),
     "vh_dequantize": (

@@ -448,43 +448,50 @@ def bake_mx8_f16(codes: torch.Tensor, scale_bytes: torch.Tensor, scale_bias: int
     return MX8F16Weight(w, e, N, K)
 
 
-def quantize_mx8_f16(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+def quantize_mx8_f16(x: torch.Tensor, as_codes: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """``quantize_mx(x, int8, [-1], 16, 127, force_scale_power_of_two=True)``
     of the rows of a bf16 ``x`` [M, K], as the exact fp16 rows ``linear_mx8_f16``
-    reads, and their exponents."""
+    reads, and their exponents; with ``as_codes`` a NaN element is the code 0
+    that ``quantize_mx_packed`` gives it."""
     if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise NotImplementedError("quantize_mx8_f16 takes a 2-D bfloat16 tensor")
     M, K = x.shape
     xc = x.contiguous()
     out = torch.empty(M, K, dtype=torch.float16, device=x.device)
     ex = torch.empty(M, dtype=torch.int32, device=x.device)
-    _lib.check(load().vh_quantize_mx8_f16(ptr(xc), M, K, ptr(out), ptr(ex), ctypes.c_void_p(stream_of(x))),
-               "vh_quantize_mx8_f16")
+    name = "vh_quantize_mx8_f16_codes" if as_codes else "vh_quantize_mx8_f16"
+    _lib.check(getattr(load(), name)(ptr(xc), M, K, ptr(out), ptr(ex), ctypes.c_void_p(stream_of(x))), name)
     return out, ex
 
 
 def mx8_f16_plan(M: int, N: int, K: int) -> Tuple[int, int]:
     """(tile, splits) of ``linear_mx8_f16``.  Measured on MI355X at K = N =
     4096, one split storing through the GEMM's own epilogue unless stated:
-    M = 2048 on 256x128 tiles 56.0 us (1226 TFLOP/s; 128x128 65.0; 256x128
-    in two splits plus the reduction 92.5); M = 256 on 64x64 tiles (two
-    waves, eight stages) 15.8 us (64x128 18.9; 64x64 in two splits plus the
-    reduction 25.9); M = 128 / 64 / 16 on 64x64 tiles in two splits 15.1 /
-    14.7 / 12.5 us (unsplit 15.7 / 15.7 / 15.5; 64x128 18.7 / 18.6 / 16.8);
-    M = 512 on 64x128 tiles 21.5 us (64x64 30.1).  So: 64x64 while its grid
-    is at most 256 workgroups, in two K splits while that grid is at most
-    128; then 64x128 below 1024 rows (K split until the grid reaches 128
-    workgroups, each split at least 512 elements); from 1024, 256x128."""
-    if M >= 1024:
-        return 3, 1
+    M = 256 on 64x64 tiles (two waves, eight stages) 15.8 us (64x128 18.9;
+    64x64 in two splits plus the reduction 25.9); M = 128 / 64 / 16 on 64x64
+    tiles in two splits 15.1 / 14.7 / 12.5 us (unsplit 15.7 / 15.7 / 15.5;
+    64x128 18.7 / 18.6 / 16.8).  So: 64x64 while its grid is at most 256
+    workgroups, in two K splits while that grid is at most 128.  Above, the
+    tile of the least estimated time, as the fp8 and bf16 GEMMs choose:
+    rounds of 256 workgroups times one tile's own time plus what a full
+    round's tiles cost each other, fitted at K = 4096 (M = 513 / 800 / 1111 /
+    2048 at K = N = 4096: 29.2 / 34.6 / 44.3 / 67 us, where a choice by rows
+    took 42.7 / 41.3 / 48.3 / 67; (4096, 14336): 83.6 / 104 / 143 / 220
+    against 101 / 126 / 163 / 232)."""
     t64 = -(-M // 64) * -(-N // 64)
     if t64 <= 256:
         return 4, (2 if t64 <= 128 and K % (2 * 512) == 0 else 1)
-    tiles = -(-M // 64) * -(-N // 128)
-    splits = 1
-    while tiles * splits < 128 and K % (splits * 2 * 512) == 0 and splits < 8:
-        splits *= 2
-    return 1, splits
+
+    def estimate(t):
+        n = -(-M // t[1]) * -(-N // t[2])
+        return -(-n // 256) * t[3] + n / 256 * t[4]
+
+    return min(_MX8_F16_TILES, key=estimate)[0], 1
+
+
+# (tile, rows, columns, us of one tile, us a full round adds)
+_MX8_F16_TILES = ((1, 64, 128, 18.1, 4.1), (0, 128, 128, 21.2, 13.3), (5, 128, 192, 26.6, 22.0),
+                  (3, 256, 128, 32.2, 27.5), (6, 256, 160, 40.5, 33.0), (7, 256, 256, 81.4, 26.9))
 
 
 def linear_mx8_f16(x16: torch.Tensor, ex: torch.Tensor, weight: MX8F16Weight, out_dtype=torch.bfloat16, bias=None,

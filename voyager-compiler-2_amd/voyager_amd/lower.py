@@ -312,7 +312,8 @@ def lowered_fp8_linear(x, x_scale, qmap, w_bytes, out_scale):
     """quantize(x, x_scale, qmap=e4m3) -> linear -> dequantize(., out_scale)
     on E4M3 bytes (at decode sizes in one launch)."""
     xr = _rows(x)
-    if (_one_launch(xr, w_bytes) and (xr.shape[0] <= 4 or xr.shape[1] <= 8192) and x_scale.dtype == torch.bfloat16 and x_scale.numel() == 1
+    if (_one_launch(xr, w_bytes) and (xr.shape[0] <= 4 or xr.shape[1] <= 8192)
+            and x_scale.dtype == torch.bfloat16 and x_scale.numel() == 1
             and formats.classify(qmap).fmt.flags & FMT_HW_E4M3):
         return gemm.linear_fp8_rows8(xr, x_scale, w_bytes, out_scale).reshape(*x.shape[:-1], w_bytes.shape[0])
     xq = packed.quantize_packed(xr, x_scale, qmap)
@@ -337,6 +338,14 @@ def lowered_mxint8_linear(x, qmap, w_codes, w_scale, w_bias, block_size: int, bi
             and w_scale.shape == (w_codes.shape[0], xr.shape[1] // 16) and w_scale.shape[1] % 4 == 0
             and w_scale.data_ptr() % 4 == 0 and f.kind == FMT_INT and (f.p0, f.p1) == (-128, 127)):
         return gemm.linear_mxint8_rows8(xr, w_codes, w_scale, w_bias, bias).reshape(*x.shape[:-1], w_codes.shape[0])
+    if (block_size == 16 and xr.dtype == torch.bfloat16 and xr.data_ptr() % 16 == 0 and f.kind == FMT_INT
+            and (f.p0, f.p1) == (-128, 127) and xr.shape[1] % 16 == 0
+            and w_scale.shape == (w_codes.shape[0], xr.shape[1] // 16)
+            and gemm.mxint8_two_pass_pays(xr.shape[0], w_codes.shape[0], xr.shape[1])):
+        # linear_mxint8's two-pass form, the activation quantized straight to its fp16 rows
+        x16, ex = gemm.quantize_mx8_f16(xr, as_codes=True)
+        y = gemm.linear_mx8_f16(x16, ex, gemm.bake_mx8_f16(w_codes.view(torch.int8), w_scale, w_bias), bias=bias)
+        return y.reshape(*x.shape[:-1], w_codes.shape[0])
     px = packed.quantize_mx_packed(xr, qmap, [-1], block_size, 127.0, True)
     y = gemm.linear_mxint8(px.codes, px.scale, w_codes, w_scale, block_size, px.bias, w_bias, bias=bias)
     return y.reshape(*x.shape[:-1], w_codes.shape[0])
