@@ -31,7 +31,7 @@ GQA = 4
 
 
 def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return ctypes.c_void_p(_lib.stream_of(t))
 
 
 class ErrorFlag:

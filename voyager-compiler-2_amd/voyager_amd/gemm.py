@@ -78,8 +78,7 @@ def plan(desc: GemmDesc):
 def run(desc: GemmDesc, device) -> None:
     if plan_log is not None:
         plan_log.append(plan(desc) + (desc.M, desc.N, desc.K))
-    st = load().vh_gemm(ctypes.c_void_p(ctypes.addressof(desc)),
-                        ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream))
+    st = load().vh_gemm(ctypes.addressof(desc), _lib.stream_on(device))
     _lib.check(st, "vh_gemm")
 
 
@@ -132,7 +131,7 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out_dtype, bias=None, alpha=None
     if b.dim() == 2 and a.dim() > 2:  # one GEMM over all leading dims
         lead = a.shape[:-1]
         return gemm_bf16(a.reshape(-1, K), b, out_dtype, bias, alpha).view(*lead, b.shape[0])
-    batch_shape = torch.broadcast_shapes(a.shape[:-2], b.shape[:-2])
+    batch_shape = torch.broadcast_shapes(a.shape[:-2], b.shape[:-2]) if a.dim() > 2 or b.dim() > 2 else ()
     M, N = a.shape[-2], b.shape[-2]
     a3 = a.expand(*batch_shape, M, K).reshape(-1, M, K).contiguous() if a.dim() > 2 else a.contiguous()
     bb = b.expand(*batch_shape, N, K) if b.dim() > 2 else b

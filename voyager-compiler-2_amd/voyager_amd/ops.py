@@ -104,8 +104,14 @@ def _param(p: Optional[torch.Tensor], shape: Sequence[int], block_size: Optional
     return prm, p
 
 
+_SHAPE_ARRS = tuple(ctypes.c_int64 * max(n, 1) for n in range(_lib.MAX_DIMS + 1))
+
+
 def _shape_arr(shape):
-    return (ctypes.c_int64 * max(len(shape), 1))(*shape) if len(shape) else (ctypes.c_int64 * 1)(1)
+    n = len(shape)
+    if n > _lib.MAX_DIMS:
+        return (ctypes.c_int64 * n)(*shape)
+    return _SHAPE_ARRS[n](*shape) if n else _SHAPE_ARRS[0](1)
 
 
 def _elementwise(kind: str, x: torch.Tensor, scale, zp, block_size, cdt, fmt_a: Optional[Format],
@@ -386,12 +392,15 @@ def _axes_list(x: torch.Tensor, axes) -> List[int]:
     """The blocked axes, non-negative and ascending (``_reshape_to_blocks``,
     ``quantization/mx_utils.py:66-80``)."""
     axes = [axes] if isinstance(axes, int) else list(axes)
+    nd = x.dim()
     out = []
     for a in axes:
-        ax = a + x.dim() if a < 0 else a
-        if not 0 <= ax < max(x.dim(), 1):
-            raise IndexError(f"axis {a} out of range for a {x.dim()}-d tensor")
+        ax = a + nd if a < 0 else a
+        if not 0 <= ax < max(nd, 1):
+            raise IndexError(f"axis {a} out of range for a {nd}-d tensor")
         out.append(ax)
+    if len(out) == 1:
+        return out
     if len(set(out)) != len(out):
         raise ValueError(f"repeated block axes {axes}")
     return sorted(out)
@@ -404,13 +413,8 @@ def _block_view(x: torch.Tensor, axes):
         raise ValueError("one block axis expected")
     ax = axes[0]
     xc = x.contiguous()
-    outer = 1
-    for n in xc.shape[:ax]:
-        outer *= n
-    inner = 1
-    for n in xc.shape[ax + 1:]:
-        inner *= n
-    return xc, ax, outer, xc.shape[ax], inner
+    shape = xc.shape
+    return xc, ax, math.prod(shape[:ax]), shape[ax], math.prod(shape[ax + 1:])
 
 
 def _scale_shape(x: torch.Tensor, ax: int, block_size: int):
@@ -593,8 +597,10 @@ def _dequantize_mx_cuda(input, scale, block_size, code=None, global_scale=None):
     if code is not None:
         out = decode_codes(input, code, scale, block_size)
     else:
-        probe = torch.empty([1] * max(input.dim(), 1), dtype=input.dtype, device="meta")
-        cdt = torch.result_type(probe, scale)
+        cdt = input.dtype
+        if scale.dtype != cdt:
+            probe = torch.empty([1] * max(input.dim(), 1), dtype=cdt, device="meta")
+            cdt = torch.result_type(probe, scale)
         out = _elementwise("dequantize", input, scale, None, block_size, cdt, None, None, cdt)
     if global_scale is not None:
         out = out * global_scale
