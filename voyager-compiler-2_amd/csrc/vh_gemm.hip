@@ -1110,12 +1110,21 @@ __device__ __forceinline__ void dma16(const i32x4& rsrc, uint32_t lds, int voff)
 }
 
 // dma16 of lanes 0..31 alone (512 bytes); the whole wave has to be active.
-__device__ __forceinline__ void dma16_half(const i32x4& rsrc, uint32_t lds, int voff) {
+__device__ __forceinline__ void dma16_half(const i32x4& rsrc, uint32_t lds, int voff, int soff) {
   asm volatile(
-      "s_mov_b32 exec_hi, 0\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds\n\ts_mov_b32 exec_hi, -1"
+      "s_mov_b32 exec_hi, 0\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds\n\ts_mov_b32 exec_hi, -1"
       :
-      : "v"(voff), "s"(rsrc), "{m0}"(lds)
+      : "v"(voff), "s"(rsrc), "{m0}"(lds), "s"(soff)
       : "memory");
+}
+
+// dma16 from rsrc + voff + soff, soff uniform.  soff has to keep every offset
+// that voff puts inside the resource inside it, and the other way round.
+__device__ __forceinline__ void dma16_at(const i32x4& rsrc, uint32_t lds, int voff, int soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
+               :
+               : "v"(voff), "s"(rsrc), "{m0}"(lds), "s"(soff)
+               : "memory");
 }
 
 // Waves per SIMD the direct-to-LDS kernel asks for: one per four waves of
@@ -2067,12 +2076,13 @@ int launch_nf4(GemmArgs g, const Nf4Args& q, int splits, float* part, hipStream_
 // + 1 are free.
 //
 // MI355X, us, the activation's decode not counted (k_gemm_nf4 beside it):
-// (K, N) = (4096, 14336) at 17 / 64 / 128 / 201 / 256 rows: 16.5 / 21.3 /
-// 32.2 / 49.5 / 53.7 (42.5 / 46.0 / 48.8 / 78.2 / 78.5); (14336, 4096): 16.9
-// / 22.6 / 31.4 / 47.4 / 50.7 (41.2 / 44.8 / 46.0 / 76.4 / 77.0).  At 201
+// (K, N) = (4096, 14336) at 17 / 64 / 128 / 201 / 256 rows: 16.9 / 21.2 /
+// 30.9 / 47.6 / 53.2 (43.0 / 46.8 / 50.5 / 80.6 / 80.1); (14336, 4096): 18.2
+// / 22.8 / 31.0 / 46.9 / 50.6 (44.1 / 46.0 / 48.6 / 81.2 / 78.2).  At 201
 // rows the x stages alone take 35 us (every workgroup reads all of x from
-// L2), the rest without them 44, of which decode and MFMAs 10 and 12; with
-// one wave per SIMD 55.
+// L2, 10.5 TB/s over the chip), the rest without them about 40; with one
+// wave per SIMD 55, with the DMA offsets in vector registers and the
+// fragments moved between stages 49.5.  LDS bank conflicts: none.
 constexpr int NF4B_BN = 64;
 constexpr int NF4B_MAX_KCS = 256;  // blocks of a K range: its scale codes lie in LDS
 
@@ -2123,19 +2133,25 @@ k_gemm_nf4_bf16(GemmArgs g, Nf4Args q, int mt, int tiles, int kcs, float* __rest
   // + wave) .. + 7, lane -> row lane / 8, stored chunk lane % 8; blocks past
   // the range's end read zeros
   const int drow = wave * 8 + (lane >> 3);
-  const int vx0 = drow * (int)g.lda + ((lane & 7) ^ swz<128>(drow & 15)) * 16 + (kb0 + kg) * 128;
-  const int vw0 = (wave * nbk + kb0 + kg) * 512 + lane * 16;
-  const int vstep = 32 * (int)g.lda;
+  // (a resource of no bytes).  A lane's rows and chunk are its offset, the
+  // block the instruction's scalar one: whatever it is, rows past M lie past
+  // the resource and the others inside it.
+  int vx[LX];
+#pragma unroll
+  for (int d = 0; d < LX; ++d)
+    vx[d] = (drow + 32 * d) * (int)g.lda + ((lane & 7) ^ swz<128>(drow & 15)) * 16;
+  const int vw = wave * nbk * 512 + lane * 16;
   auto x_in = [&](int s, int buf) {
-    const bool live = s * KG + kg < nk;
+    const int b = s * KG + kg;
+    const i32x4 r = {ra.x, ra.y, b < nk ? ra.z : 0, ra.w};
 #pragma unroll
     for (int d = 0; d < LX; ++d)
-      dma16(ra, lds_x + buf * (KG * XB) + (4 * d + wave) * 1024,
-            live ? vx0 + d * vstep + s * (KG * 128) : (int)0x80000000);
+      dma16_at(r, lds_x + buf * (KG * XB) + (4 * d + wave) * 1024, vx[d], (kb0 + (b < nk ? b : 0)) * 128);
   };
   auto w_in = [&](int s, int buf) {
-    const bool live = s * KG + kg < nk;
-    dma16_half(rb, lds_w + buf * (KG * WB) + wave * 512, live ? vw0 + s * (KG * 512) : (int)0x80000000);
+    const int b = s * KG + kg;
+    const i32x4 r = {rb.x, rb.y, b < nk ? rb.z : 0, rb.w};
+    dma16_half(r, lds_w + buf * (KG * WB) + wave * 512, vw, (kb0 + (b < nk ? b : 0)) * 512);
   };
 
 #pragma unroll
@@ -2170,7 +2186,6 @@ k_gemm_nf4_bf16(GemmArgs g, Nf4Args q, int mt, int tiles, int kcs, float* __rest
   uint2 w[TN];           // records of the stage to decode next
   uint32_t sc_code[TN];  // scale codes of the stage after it
   float scale[TN];       // its scales
-  uint4 wf[TN][2];       // fragments of the stage to multiply
   // x fragment k of a stage: row tile k % TM, half k / TM of the block's MFMAs
   auto fragment = [&](const uint8_t* xb, int k) {
     return *(const bf16x8*)(xb + (k % TM) * 2048 + (((2 * c4 + k / TM) ^ fsw) << 4));
@@ -2182,6 +2197,7 @@ k_gemm_nf4_bf16(GemmArgs g, Nf4Args q, int mt, int tiles, int kcs, float* __rest
       scale[j] = s_sb[sc_code[j]];
     }
   };
+  uint4 wa[TN][2], wb[TN][2];  // fragments of the stage to multiply and of the next
   wait_vmcnt<0>();
   __syncthreads();
 #pragma unroll
@@ -2192,11 +2208,10 @@ k_gemm_nf4_bf16(GemmArgs g, Nf4Args q, int mt, int tiles, int kcs, float* __rest
     sc_code[j] = code(1, j);
     const uint32_t l[4] = {lut_lo(w[j].x, base, q.lvb), lut_lo(w[j].y, base, q.lvb),
                            lut_hi(w[j].x, base, q.lvb), lut_hi(w[j].y, base, q.lvb)};
-    nf4_pack16(l, scale[j], wf[j][0], wf[j][1]);
+    nf4_pack16(l, scale[j], wa[j][0], wa[j][1]);
   }
-  const int ns = (nk + KG - 1) / KG;
   int xbuf = 0, wbuf = 0;
-  for (int s = 0; s < ns; ++s) {
+  auto stage = [&](int s, uint4 (&wf)[TN][2], uint4 (&nxt)[TN][2]) {
     wait_vmcnt<(NX - 2) * L + 1>();
     lds_barrier();
     x_in(s + NX - 1, xbuf == 0 ? NX - 1 : xbuf - 1);
@@ -2241,10 +2256,16 @@ k_gemm_nf4_bf16(GemmArgs g, Nf4Args q, int mt, int tiles, int kcs, float* __rest
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      wf[j][0] = make_uint4(nf[j][0], nf[j][1], nf[j][2], nf[j][3]);
-      wf[j][1] = make_uint4(nf[j][4], nf[j][5], nf[j][6], nf[j][7]);
+      nxt[j][0] = make_uint4(nf[j][0], nf[j][1], nf[j][2], nf[j][3]);
+      nxt[j][1] = make_uint4(nf[j][4], nf[j][5], nf[j][6], nf[j][7]);
     }
     xbuf = xbuf == NX - 1 ? 0 : xbuf + 1;
+  };
+  // in pairs, so that the fragments change places without moves (a stage
+  // past the end multiplies zeros)
+  for (int s = 0; s * KG < nk; s += 2) {
+    stage(s, wa, wb);
+    stage(s + 1, wb, wa);
   }
   wait_vmcnt<0>();
 

@@ -728,8 +728,8 @@ def nf4_two_pass_pays(M: int, N: int, K: int) -> bool:
     weight block once per 256 rows and multiplies at half the bf16 GEMM's
     rate.  Measured on MI355X (``vh_gemm_nf4_bf16`` with the activation's
     decode / two-pass, us): (K, N) = (4096, 4096) at M = 256: 29.6 / 32.5,
-    300: 32.0 / 32.7, 512: 39.1 / 34.2; (4096, 14336): 57.5 / 58.9, 84.2 /
-    72.1, 103 / 77.9; (14336, 4096): 55.5 / 87.3, 73.5 / 94.7, 99.9 / 102;
+    300: 31.2 / 32.9, 512: 39.1 / 34.2; (4096, 14336): 57.0 / 61.8, 80.1 /
+    74.1, 103 / 77.9; (14336, 4096): 55.4 / 87.8, 68.0 / 91.5, 99.9 / 102;
     (4096, 1024): 25.8 / 26.8, 21.8 / 30.5, 24.5 / 30.5.  So up to 256 rows
     the one tile of rows decides, and above them only columns too few to
     fill the chip do.  The two-pass form holds the decoded weight (2 bytes
