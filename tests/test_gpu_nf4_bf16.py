@@ -66,3 +66,47 @@ def test_nf4_quantize_bf16(M, K):
     xo, _ = gemm.nf4_decode_bf16(px, wb, decode_w=False)
     got = gemm.nf4_quantize_bf16(x, wb, formats.classify(index), formats.classify(stab))
     assert_same_bits(got, xo)
+
+
+@pytest.mark.parametrize("form", ["plain", "misaligned", "strided", "transposed", "float32", "float16"])
+@pytest.mark.parametrize("M,K,N", [(17, 4096, 2064), (190, 1088, 4112), (320, 640, 2048), (300, 704, 2064)])
+def test_linear_nf4_routes(form, M, K, N):
+    """Every form of activation ``linear_nf4`` takes above 16 rows, on the
+    route it chooses, against the fused kernel (the bound of
+    ``test_gemm_nf4_bf16`` for each of the two sums), eagerly and from a
+    replayed graph."""
+    from voyager_amd import gemm, packed
+
+    index, entries, stab = _maps()
+    g = torch.Generator().manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    w = (torch.randn(N, K, generator=g) * 0.02).bfloat16().cuda()
+    if form == "misaligned":
+        x = torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(M, K)
+        assert x.data_ptr() % 16
+    elif form == "strided":
+        x = torch.stack([x, x], 2).reshape(M, 2 * K)[:, ::2]
+    elif form == "transposed":
+        x = x.t().contiguous().t()
+    elif form != "plain":
+        x = x.to(getattr(torch, form))
+    wb = gemm.bake_nf4_weight(w, index, stab, entries)
+    px = packed.quantize_mx_packed(x.contiguous(), index, [-1], 64, 31.0, False, stab)
+    xo, wo = gemm.nf4_decode_bf16(px, wb)
+    bound = 2 * K * 2.0**-24 * (xo.double().abs() @ wo.double().abs().T)
+    ref = gemm.linear_nf4_prefill(x, wb, index, stab, torch.float32, tile=1, two_pass=False)
+
+    def call():
+        return gemm.linear_nf4(x, wb, index, stab, torch.float32)
+
+    got = call()
+    assert ((got - ref).double().abs() <= bound).all()
+    assert torch.equal(gemm.gemm_nf4_packed(px, wb, torch.float32), got)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, call())
