@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import voyager_amd.library  # noqa: F401  (defines quantized_ops)
-from helpers import max_rel_err
+from helpers import assert_same_bits, max_rel_err
 from voyager_amd import formats, gemm, lower, packed
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +77,33 @@ def test_skinny_mxint8(M, N, K):
     assert ((y.double() - ref).abs() <= room).all()
     assert torch.equal(lower.lowered_mxint8_linear(x, tab, pw.codes, pw.scale, pw.bias, 16, bias),
                        gemm.linear_mxint8(*args, bias=bias))
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 40, 528), (8, 4104, 4160), (20, 100, 4112), (33, 56, 1040)])
+def test_skinny_mxint8_padded_rows(M, N, K):
+    """Codes and scale bytes as columns of wider tensors, the scale views
+    ending where their storage does (or one to three bytes before, as their
+    rows are 4-byte aligned): the contiguous operands' bits, also where a
+    group's scales go past the row's end and hold the next row's."""
+    x, w = _inputs(M, N, K)
+    tab = formats.quantization_map("int8")
+    px, pw = (packed.quantize_mx_packed(t, tab, [-1], 16, 127.0, True) for t in (x, w))
+
+    def padded(t, at, unit):
+        pitch = -(-(at + t.shape[1]) // unit) * unit
+        wide = torch.full((t.shape[0], pitch), 0x7f, dtype=t.dtype, device="cuda")
+        view = wide[:, at:at + t.shape[1]]
+        view.copy_(t)
+        return view
+
+    flat = gemm.linear_mxint8(px.codes, px.scale, pw.codes, pw.scale, 16, px.bias, pw.bias)
+    args = [f(p) for p in (px, pw) for f in (lambda p: padded(p.codes, 16, 16), lambda p: padded(p.scale, 4, 4))]
+    y, log = _log(lambda: gemm.linear_mxint8(*args, 16, px.bias, pw.bias))
+    assert [p[0] for p in log] == [gemm.FAMILY_SKINNY]
+    assert_same_bits(y, flat)
+    if M <= 8:
+        one = lower.lowered_mxint8_linear(x, tab, args[2], args[3], pw.bias, 16)
+        assert_same_bits(one, flat)
 
 
 @pytest.mark.parametrize("M,N,K", [s for s in SHAPES if s[2] % 8 == 0] + [(2, 7, 24)])

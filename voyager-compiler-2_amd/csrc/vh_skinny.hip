@@ -218,8 +218,12 @@ __global__ void __launch_bounds__(WAVES * 64) k_skinny(SkinnyArgs g) {
   const rsrc_t ra = rsrc(g.A + bat * g.sa, g.M * g.lda);
   rsrc_t rbs = rb, ras = ra;
   if constexpr (FMT == OP_MXI8) {
-    rbs = rsrc(g.b_scale + n0 * g.lds_b, rows_b * g.lds_b);
-    if constexpr (!FUSED) ras = rsrc(g.a_scale, (int64_t)g.M * g.lds_a);
+    // A group's scale bytes go past a row's end where K is no whole group:
+    // the resource ends with the last row's own (in whole dwords, as the
+    // pitch is), since a padded view's storage may end there too.
+    const int64_t last = (g.K / 16 + 3) & ~3;
+    rbs = rsrc(g.b_scale + n0 * g.lds_b, (rows_b - 1) * g.lds_b + last);
+    if constexpr (!FUSED) ras = rsrc(g.a_scale, (int64_t)(g.M - 1) * g.lds_a + last);
   }
 
   struct Set {
