@@ -2508,34 +2508,41 @@ int staged_tile(int c) {
 // so T tiles take ceil(T / 256) rounds of one tile's own time (c0: its MFMAs
 // and fill) plus what the running tiles cost each other in L2, HBM and clock
 // (c1 a full round's worth); the tile of the least sum is taken.  c0 and c1
-// are least-squares fits in us at K = 4096 (K scales both alike) over M =
-// 201 .. 2048 on MI355X at (K, N) = (4096, 4096), (4096, 14336), (14336,
-// 4096), every tile timed at every size; over those 36 sizes the choice is
-// within 4% of the best tile.  A choice by thresholds on the tile count
-// alone left rounds nearly empty: fp8 at M = 513 / 1111 / 1300, K = N = 4096
-// 24.6 / 32.2 / 33.3 us against 17.4 / 23.8 / 25.9 (bf16 39.1 / 54.7 / 55.4
-// against 27.2 / 40.4 / 45.3); (4096, 14336) at M = 513 / 1111 / 2048 52.9 /
-// 82.6 / 106.8 against 43.7 / 68.7 / 106.6 (bf16, M = 513 / 1111, 94.8 / 150
-// against 76.5 / 128).
+// are least-squares fits in us at K = 4096 over M = 201 .. 2048 on MI355X at
+// (K, N) = (4096, 4096), (4096, 14336), (14336, 4096), every tile timed at
+// every size; over those 36 sizes the choice is within 4% of the best tile.
+// A choice by thresholds on the tile count alone left rounds nearly empty:
+// fp8 at M = 513 / 1111 / 1300, K = N = 4096 24.6 / 32.2 / 33.3 us against
+// 17.4 / 23.8 / 25.9 (bf16 39.1 / 54.7 / 55.4 against 27.2 / 40.4 / 45.3);
+// (4096, 14336) at M = 513 / 1111 / 2048 52.9 / 82.6 / 106.8 against 43.7 /
+// 68.7 / 106.6 (bf16, M = 513 / 1111, 94.8 / 150 against 76.5 / 128).
+// Below K = 4096 a tile's own time falls only to f, its launch, fill and
+// store, so short products want fewer, larger tiles (f fitted at K = 256 ..
+// 2048, N = 512 .. 14336, M = 65 .. 8192): with c0 scaled by K alone, as
+// before, the mean over those 528 sizes was 1.8% above the best tile (fp8;
+// bf16 1.7%) and up to 47%, now 0.2% (0.6%) and 13% (19%), one bf16 size of
+// K = 256 apart (M = 8192, N = 1024: 42%).  fp8 at K = 512, M = 4096, N = 2816
+// / 14336 23.6 / 78.8 -> 16.0 / 66.8 us.
 struct DlTile {
   int tile, bm, bn;
-  float c0, c1;
+  float f, c0, c1;
 };
-constexpr DlTile DL_FP8[] = {{37, 64, 128, 10.0f, 1.8f},   {33, 128, 128, 12.4f, 5.0f},
-                             {25, 128, 192, 15.8f, 8.1f},  {31, 256, 128, 18.8f, 10.8f},
-                             {26, 256, 160, 23.2f, 12.6f}, {44, 256, 224, 41.0f, 11.2f},
-                             {41, 256, 256, 42.1f, 15.6f}};
-constexpr DlTile DL_BF16[] = {{35, 128, 64, 17.2f, 3.4f},   {33, 128, 128, 21.2f, 10.3f},
-                              {25, 128, 192, 27.8f, 15.9f}, {31, 256, 128, 33.1f, 21.6f},
-                              {26, 256, 160, 40.0f, 24.6f}, {41, 256, 256, 85.0f, 23.2f}};
+constexpr DlTile DL_FP8[] = {{37, 64, 128, 3.7f, 10.0f, 1.8f},   {33, 128, 128, 5.3f, 12.4f, 5.0f},
+                             {25, 128, 192, 6.9f, 15.8f, 8.1f},  {31, 256, 128, 8.1f, 18.8f, 10.8f},
+                             {26, 256, 160, 9.4f, 23.2f, 12.6f}, {44, 256, 224, 10.1f, 41.0f, 11.2f},
+                             {41, 256, 256, 8.8f, 42.1f, 15.6f}};
+constexpr DlTile DL_BF16[] = {{35, 128, 64, 3.2f, 17.2f, 3.4f},   {33, 128, 128, 4.4f, 21.2f, 10.3f},
+                              {25, 128, 192, 6.4f, 27.8f, 15.9f}, {31, 256, 128, 7.2f, 33.1f, 21.6f},
+                              {26, 256, 160, 8.1f, 40.0f, 24.6f}, {41, 256, 256, 5.9f, 85.0f, 23.2f}};
 
 template <int NT>
-int dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t batch) {
+int dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const float k = K < 4096 ? (float)K / 4096.0f : 1.0f;  // (from there on every term grows alike)
   int best = t[0].tile;
   float least = 0.0f;
   for (int i = 0; i < NT; ++i) {
     const int64_t n = ((M + t[i].bm - 1) / t[i].bm) * ((N + t[i].bn - 1) / t[i].bn) * batch;
-    const float us = (float)((n + 255) / 256) * t[i].c0 + (float)n / 256.0f * t[i].c1;
+    const float us = (float)((n + 255) / 256) * (t[i].f + k * (t[i].c0 - t[i].f)) + (float)n / 256.0f * k * t[i].c1;
     if (i == 0 || us < least) best = t[i].tile, least = us;
   }
   return best;
@@ -2570,7 +2577,7 @@ Plan plan_gemm(const vh_gemm_desc* d) {
   // validated a multiple of 16 below, where the descriptor is checked).
   const bool chunks_ok = d->lda % 16 == 0 && d->ldb % 16 == 0 && d->K % (fp8 ? 16 : 8) == 0;
   if (fp8 && dl_ok && chunks_ok) {
-    const int c = d->tile_hint ? d->tile_hint : dl_tile(DL_FP8, d->M, d->N, batch);
+    const int c = d->tile_hint ? d->tile_hint : dl_tile(DL_FP8, d->M, d->N, d->K, batch);
     if (is_direct_fp8_tile(c)) return {FAM_DIRECT_FP8, c, 1};
   }
   if (fp8) return {FAM_STAGED, staged, 1};
@@ -2580,7 +2587,7 @@ Plan plan_gemm(const vh_gemm_desc* d) {
     // 14336 alone, but even within a run of other kernels.
     const int c = d->tile_hint ? d->tile_hint
                   : tiles(256, 256) >= 384 ? 41
-                                           : dl_tile(DL_BF16, d->M, d->N, batch);
+                                           : dl_tile(DL_BF16, d->M, d->N, d->K, batch);
     if (is_direct_bf16_tile(c)) return {FAM_DIRECT_BF16, c, 1};
   }
   if (d->a_fmt == OP_MXI8 && d->b_fmt == OP_MXI8) {
