@@ -296,12 +296,17 @@ int64_t vh_gemm_workspace_bytes(const vh_gemm_desc* desc);
  * register-staged kernel (tiles 2..10 as tile_hint names them), 2 the
  * direct-to-LDS kernel on E4M3 operands (tiles 20..48), 3 the direct-to-LDS
  * kernel on bf16 operands (25, 26, 31, 33, 35, 37, 41), 4 the MX-int8 kernels
- * (50..56) with `splits` K splits.  No counterpart in the reference, whose
+ * (50..56) with `splits` K splits, 5 the few-row kernel (at most 64 rows, E4M3,
+ * bf16 or MX-int8 of 16-element blocks; tile 0, one split, no workspace), which
+ * runs without a hint where it is the faster one and with tile_hint
+ * VH_GEMM_TILE_SKINNY where it can.  No counterpart in the reference, whose
  * GEMM is one aten call; tests use it to assert which tile a shape takes. */
 #define VH_GEMM_FAMILY_STAGED 1
 #define VH_GEMM_FAMILY_DIRECT_FP8 2
 #define VH_GEMM_FAMILY_DIRECT_BF16 3
 #define VH_GEMM_FAMILY_MXI8 4
+#define VH_GEMM_FAMILY_SKINNY 5
+#define VH_GEMM_TILE_SKINNY 70
 int vh_gemm_plan(const vh_gemm_desc* desc, int32_t* family, int32_t* tile, int32_t* splits);
 
 /* ------------------------------------------------------------ MXNF4 GEMV

@@ -42,3 +42,27 @@ def test_direct_tiles(fmt, M, N, K, tile):
                                         (1111, 4096, 14336, 5), (2048, 4096, 4096, 3), (2048, 14336, 4096, 7)])
 def test_fp16_row_tiles(M, N, K, tile):
     assert gemm.mx8_f16_plan(M, N, K) == (tile, 1)
+
+
+# (rows, N, K, batch): the few-row kernel or the tiles
+FEW_ROWS = {
+    gemm.OP_BF16: {True: [(1, 4096, 64, 1), (64, 4096, 64, 1), (16, 8192, 128, 1), (32, 8192, 2048, 1),
+                          (64, 8192, 2048, 1), (16, 14336, 2048, 1), (32, 14336, 4096, 1), (16, 32768, 4096, 1), (16, 512, 512, 8),
+                          (17, 256, 128, 8), (64, 128, 128, 8), (32, 1024, 4096, 32), (33, 1024, 2048, 4)],
+                   False: [(32, 8192, 128, 1), (64, 8192, 512, 1), (1, 14336, 512, 1), (64, 14336, 4096, 1),
+                           (1, 32768, 1024, 1), (16, 20480, 4096, 1), (65, 4096, 4096, 1), (1, 4096, 128, 256),
+                           (16, 1024, 128, 256), (32, 1024, 512, 32), (32, 512, 128, 8), (64, 64, 2048, 64)]},
+    gemm.OP_FP8: {True: [(1, 4096, 64, 1), (64, 4096, 512, 1), (16, 8192, 512, 1), (32, 14336, 4096, 1)],
+                  False: [(32, 8192, 512, 1), (1, 14336, 1024, 1), (64, 14336, 4096, 1), (1, 20480, 4096, 1),
+                          (16, 32768, 14336, 1)]},
+    gemm.OP_MXI8: {True: [(16, 4096, 128, 1), (32, 14336, 256, 1), (64, 4096, 4096, 1), (1, 65536, 512, 1)],
+                   False: [(16, 4096, 64, 1), (17, 4096, 128, 1), (64, 4112, 4096, 1), (1, 28672, 256, 1)]},
+}
+
+
+@pytest.mark.parametrize("fmt,few,M,N,K,batch", [(f, few) + c for f, d in FEW_ROWS.items() for few, cs in d.items()
+                                                 for c in cs])
+def test_few_rows(fmt, few, M, N, K, batch):
+    assert (_plan(fmt, M, N, K, batch)[0] == gemm.FAMILY_SKINNY) == few
+    if M <= 64:
+        assert _plan(fmt, M, N, K, batch, gemm.TILE_SKINNY)[0] == gemm.FAMILY_SKINNY

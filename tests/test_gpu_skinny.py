@@ -1,8 +1,9 @@
 """GEMMs of at most 64 rows (``k_skinny``) and the lowered linears that
 quantize at most 8 rows in the same launch: at the edges of the row tiles
 (16, 32, 64), of the weight tiles (16 rows; 1, 2 or 4 of them a workgroup) and
-of K (one chunk, part of a group, fewer groups than waves), against the exact
-product of the decoded operands and, bit for bit, one launch against two."""
+of K (one chunk, part of a group, fewer groups than waves, several groups a
+wave and part of one), against the exact product of the decoded operands and,
+bit for bit, one launch against two."""
 
 import pytest
 import torch
@@ -16,6 +17,11 @@ pytestmark = pytest.mark.gpu
 # (M, N, K): N around 16 and past one and two rounds of 256 tiles
 SHAPES = [(1, 16, 16), (3, 40, 528), (4, 1000, 4096), (8, 4104, 272), (16, 8200, 1040), (17, 100, 4096),
           (32, 4112, 64), (33, 1048, 2064), (64, 8192, 512), (5, 14336, 320)]
+# MX-int8 decodes in the kernel and holds scales beside the codes: every row
+# tile and weight tile with several groups a wave and part of one at the end
+MX_SHAPES = [s for s in SHAPES if s[2] % 64 == 0] + [
+    (3, 4112, 4160), (7, 1000, 4160), (8, 4104, 4160), (16, 4112, 4160), (16, 8200, 4160), (17, 1000, 4160),
+    (32, 4112, 4160), (32, 8208, 4160), (33, 1048, 4032), (64, 4096, 4032)]
 
 
 def _inputs(M, N, K):
@@ -43,7 +49,7 @@ def test_skinny_fp8(M, N, K):
     tab = formats.quantization_map("fp8_e4m3")
     sx = torch.tensor(0.013, dtype=torch.bfloat16, device="cuda")
     xq, wq = packed.quantize_packed(x, sx, tab), packed.quantize_packed(w, sx, tab)
-    y, log = _log(lambda: gemm.linear_fp8(xq, wq, sx))
+    y, log = _log(lambda: gemm.linear_fp8(xq, wq, sx, tile_hint=gemm.TILE_SKINNY))
     assert [p[0] for p in log] == [gemm.FAMILY_SKINNY]
     vx, vw = packed.unpack_codes(xq, tab).double(), packed.unpack_codes(wq, tab).double()
     # the FP8 MFMA rounds the products it adds at once to a common grid (3.2e-4
@@ -53,10 +59,10 @@ def test_skinny_fp8(M, N, K):
     room = vx.abs() @ vw.abs().T * sx.double() * 2.0**-11 + exp.abs() * 2.0**-7
     assert ((y.double() - exp).abs() <= room).all()
     one = lower.lowered_fp8_linear(x, sx, tab, wq, sx)
-    assert torch.equal(one, y)
+    assert torch.equal(one, y if M <= 8 else gemm.linear_fp8(xq, wq, sx))
 
 
-@pytest.mark.parametrize("M,N,K", [s for s in SHAPES if s[2] % 64 == 0])
+@pytest.mark.parametrize("M,N,K", MX_SHAPES)
 def test_skinny_mxint8(M, N, K):
     x, w = _inputs(M, N, K)
     tab = formats.quantization_map("int8")
@@ -68,15 +74,15 @@ def test_skinny_mxint8(M, N, K):
 
     args = (px.codes, px.scale, pw.codes, pw.scale, 16, px.bias, pw.bias)
     alpha, bias = torch.tensor(0.75, device="cuda"), torch.randn(N, device="cuda").bfloat16()
-    y, log = _log(lambda: gemm.linear_mxint8(*args, out_dtype=torch.float32, bias=bias, alpha=alpha))
-    small = M <= 32 or (N <= 4096 and K <= 4096)
-    assert [p[0] for p in log] == [gemm.FAMILY_SKINNY if small else gemm.FAMILY_MXI8]
+    y, log = _log(lambda: gemm.linear_mxint8(*args, out_dtype=torch.float32, bias=bias, alpha=alpha,
+                                             tile_hint=gemm.TILE_SKINNY))
+    assert [p[0] for p in log] == [gemm.FAMILY_SKINNY]
     ref = value(px) @ value(pw).T * 0.75 + bias.double()
     # exact products; float32 sums of K terms, each rounded
     room = value(px).abs() @ value(pw).abs().T * 0.75 * K * 2.0**-24 + ref.abs() * 2.0**-22
     assert ((y.double() - ref).abs() <= room).all()
     assert torch.equal(lower.lowered_mxint8_linear(x, tab, pw.codes, pw.scale, pw.bias, 16, bias),
-                       gemm.linear_mxint8(*args, bias=bias))
+                       gemm.linear_mxint8(*args, bias=bias, tile_hint=gemm.TILE_SKINNY if M <= 8 else 0))
 
 
 @pytest.mark.parametrize("M,N,K", [(3, 40, 528), (8, 4104, 4160), (20, 100, 4112), (33, 56, 1040)])
@@ -111,14 +117,19 @@ def test_skinny_mxint8_padded_rows(M, N, K):
 def test_skinny_bf16(M, N, K, out_dtype):
     x, w = _inputs(M, N, K)
     x = x.clamp(-10, 10)
-    y, log = _log(lambda: torch.ops.quantized_ops.linear(x, w, out_dtype=out_dtype))
+    y, log = _log(lambda: gemm.gemm_bf16(x, w, out_dtype, tile_hint=gemm.TILE_SKINNY))
     assert [p[0] for p in log] == [gemm.FAMILY_SKINNY]
     ref = x.double() @ w.double().T
-    assert max_rel_err(y, ref) < (2.0**-8 if out_dtype == torch.bfloat16 else 1e-5)
+    room = 2.0**-8 if out_dtype == torch.bfloat16 else 1e-5
+    assert max_rel_err(y, ref) < room
+    assert max_rel_err(torch.ops.quantized_ops.linear(x, w, out_dtype=out_dtype), ref) < room
     # a batch of products, the rows' tiles of each its own
     xb, wb = torch.stack([x, 2 * x]), torch.stack([w, w * 0.5])
+    yb, log = _log(lambda: gemm.gemm_bf16(xb, wb, out_dtype, tile_hint=gemm.TILE_SKINNY))
+    assert [p[0] for p in log] == [gemm.FAMILY_SKINNY]
+    assert max_rel_err(yb, torch.stack([ref, ref])) < room
     yb = torch.ops.quantized_ops.matmul(xb, wb, layout="xc,kc->xk", out_dtype=out_dtype)
-    assert max_rel_err(yb, torch.stack([ref, ref])) < (2.0**-8 if out_dtype == torch.bfloat16 else 1e-5)
+    assert max_rel_err(yb, torch.stack([ref, ref])) < room
 
 
 def test_rows8_nan_and_infinity():

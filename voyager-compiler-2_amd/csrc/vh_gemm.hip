@@ -2556,7 +2556,7 @@ Plan plan_gemm(const vh_gemm_desc* d) {
   auto tiles = [&](int bm, int bn) { return ((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn) * batch; };
   const bool fp8 = d->a_fmt == OP_FP8;
   const bool dl_ok = f8dl_epilogue_ok(d->C, d->epi.out_dtype, d->ldc, d->N);
-  if (vh::skinny_fits(d)) return {FAM_SKINNY, 0, 1};
+  if (vh::skinny_taken(d)) return {FAM_SKINNY, 0, 1};
   // Register-staged kernel (bf16, MX-int8 and posit8 operands; fp8 when the
   // LDS epilogue does not apply).  Measured on MI355X at M = 2048 with fp8
   // data (K in {4096, 14336}, N in {1024, 4096, 14336}): 8-wave blocks (two
@@ -2644,6 +2644,8 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
     if (fmt == OP_P8) VH_REQUIRE(d->lut, "vh_gemm: posit8 operand needs its decode table");
   }
   VH_REQUIRE(d->lda * 256 < (1ll << 31) && d->ldb * 256 < (1ll << 31), "vh_gemm: rows too long for 32-bit offsets");
+  VH_REQUIRE(d->tile_hint != VH_GEMM_TILE_SKINNY || vh::skinny_fits(d),
+             "vh_gemm: the few-row kernel cannot take this product");
   if (d->M == 0 || d->N == 0) return VH_OK;
   GemmArgs g;
   memset(&g, 0, sizeof(g));
@@ -2755,7 +2757,7 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
 }
 
 extern "C" int64_t vh_gemm_workspace_bytes(const vh_gemm_desc* d) {
-  if (!d || vh::skinny_fits(d)) return 0;
+  if (!d || vh::skinny_taken(d)) return 0;
   int cfg, splits;
   mxi8_plan(d, cfg, splits);
   return cfg ? mxi8_workspace(d, splits) : 0;

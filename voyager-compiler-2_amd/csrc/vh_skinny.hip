@@ -556,27 +556,65 @@ SkinnyArgs rows8_args(const uint16_t* x, int64_t ldx, const uint8_t* w, int64_t 
 namespace vh {
 
 bool skinny_fits(const vh_gemm_desc* d) {
-  // Measured on MI355X, weights from HBM (this kernel / the tiled ones, us),
-  // (K, N) = (4096, 4096), (4096, 1024), (4096, 14336), (14336, 4096):
-  //   E4M3     16 rows   7.1 / 14.8   6.2 / 14.2  15.4 / 17.8  14.6 / 43.5
-  //            64       10.5 / 17.2   9.2 / 16.7  23.3 / 21.1  25.3 / 53.1
-  //   bf16     16       10.1 / 21.8   8.1 / 21.1  26.1 / 29.8  27.6 / 68.3
-  //            64       15.5 / 23.4  13.9 / 22.5  37.6 / 30.1  46.3 / 75.0
-  //   MX-int8  16        9.6 / 16.0   8.6 / 18.3  20.3 / 33.9  19.9 / 30.5
-  //            32       12.3 / 17.0  11.2 / 17.9  23.6 / 35.3  27.0 / 32.4
-  //            64       16.5 / 19.7  15.5 / 19.8  57.7 / 38.9  41.2 / 32.4
-  // (MX-int8 with its split reduction).  Past 32 rows a second round of wide
-  // weights, and MX-int8's decode of the activation, cost more than the tiles.
-  if (d->M > MAX_ROWS || d->tile_hint != 0 || d->split_k != 0 || d->a_fmt != d->b_fmt) return false;
-  if (d->M > 32 && (d->a_fmt == OP_MXI8 ? d->N > 4096 || d->K > 4096 : d->N * (d->batch < 1 ? 1 : d->batch) > 8192))
-    return false;
-  if (d->lda % 16 || d->ldb % 16 || d->K <= 0) return false;
+  if (d->M > MAX_ROWS || d->a_fmt != d->b_fmt || d->lda % 16 || d->ldb % 16 || d->K <= 0) return false;
   if (d->a_fmt == OP_FP8 || d->a_fmt == OP_BF16) return true;
   if (d->a_fmt != OP_MXI8) return false;
   auto al = [](const void* p, int64_t ld) { return (uintptr_t)p % 4 == 0 && ld % 4 == 0; };
   return d->batch <= 1 && d->a_block == 16 && d->b_block == 16 && d->K % 16 == 0 && bias_ok(d->a_bias) &&
          bias_ok(d->b_bias) && al(d->a_scale, d->a_scale_ld) && al(d->b_scale, d->b_scale_ld) &&
          d->a_scale_ld < (1 << 20) && d->b_scale_ld < (1 << 20);
+}
+
+bool skinny_taken(const vh_gemm_desc* d) {
+  // Measured on MI355X, weights from HBM: this kernel / the tiled ones in us (*
+  // where those are taken).
+  //                    K   N = 4096                   14336                      32768
+  //                        16 rows       64           16            64           16            64
+  //   E4M3           512    4.0 /  4.8    4.8 /  5.0    5.2 /  5.1*   9.1 /  5.3*   9.3 /  6.4*  16.9 /  7.1*
+  //                 2048    4.9 /  7.3    6.5 /  7.7    9.2 /  9.9   13.8 /  9.3*  16.9 / 13.7*  26.9 / 14.4*
+  //                 4096    6.8 / 12.2    9.7 / 15.2   12.9 / 13.0   19.2 / 13.7*  26.1 / 22.7*  39.4 / 24.1*
+  //                14336   12.6 / 27.9   19.1 / 32.3   31.6 / 32.9   42.3 / 36.2*
+  //   bf16           512    4.2 /  5.2    5.2 /  5.4    6.7 /  6.6*  11.5 /  7.0*  12.4 /  9.6*  22.0 / 10.5*
+  //                 2048    7.1 / 13.0   10.2 / 13.7   15.7 / 16.6   23.4 / 17.4*  31.9 / 34.5*  46.1 / 35.3*
+  //                 4096   10.1 / 22.2   15.9 / 23.6   26.4 / 29.1   37.8 / 30.7*  55.7 / 61.6   76.4 / 62.7*
+  //                14336   26.5 / 69.0   46.8 / 75.7   80.0 / 94.2    118 /  100*
+  //   MX-int8        128    4.3 /  5.3    5.4 /  5.4*   5.5 /  6.0   17.3 /  6.2*   9.2 / 10.4*  32.7 / 11.1*
+  //                  512    4.7 /  9.2    5.9 / 10.9    6.2 / 11.4   18.3 / 16.1*  11.3 / 17.2   34.8 / 17.9*
+  //                 4096    9.2 / 15.9   15.8 / 19.2   18.4 / 33.4   53.2 / 36.0*  36.3 / 75.8    111 / 77.7*
+  //                14336   18.8 / 30.8   37.1 / 31.9*  41.5 / 95.7    135 / 98.0*
+  //   batches of bf16      1 row         16           32            64
+  //   256 of (1024, 128)    47.1 / 31.0*  48.2 / 31.9*  54.9 / 33.1*   103 / 36.2*
+  //   32 of (1024, 512)     12.4 /  9.8*  12.9 /  9.9*  14.5 / 10.4*  22.4 / 11.7*
+  //   8 of (512, 512)        4.2 /  5.2    4.3 /  5.2    4.8 /  5.3*   5.5 /  5.5*
+  //   32 of (1024, 4096)    54.1 / 68.0   56.3 / 68.0   58.4 / 68.2   80.6 / 70.0*
+  // One round of the CUs at NT = 1 (256 weight tiles) pays at any K; a second
+  // set of columns or a second round repeats each workgroup's latency and sum
+  // (about 2 us) and needs a K whose stream covers it; from a third on the
+  // last round has to be nearly full as well, and E4M3's tiles, twice as fast
+  // as bf16's, are then even or better.  More rows cost this kernel more than
+  // the tiles, most of all in a batch, whose every product has its own.  Over
+  // 7035 sizes (K = 64 .. 14336, N = 64 .. 65536, 1 .. 64 rows, batches of 1
+  // .. 256) the choice is 0.6% above the faster kernel on average; any K and,
+  // to 32 rows, any grid, as before, 9.7%.
+  if (d->tile_hint == VH_GEMM_TILE_SKINNY) return skinny_fits(d);
+  if (d->tile_hint != 0 || d->split_k != 0 || !skinny_fits(d)) return false;
+  const int64_t batch = d->batch < 1 ? 1 : d->batch, K = d->K, N = d->N;
+  const int64_t t = (N + 15) / 16 * batch;  // tiles of 16 weight rows
+  const bool many = d->M > 16, most = d->M > 32;
+  if (d->a_fmt == OP_MXI8) {
+    if (most && (N > 4096 || K > 4096)) return false;
+    return K >= (t > 4 * CUS ? 512 : many ? 256 : 128);
+  }
+  if (K < 2048) {
+    if (t <= CUS) return batch == 1 || t <= (most ? 64 : many ? 128 : CUS);
+    return t <= 2 * CUS && !many;
+  }
+  if (t <= CUS) return !most || batch == 1 || N >= 512 || t <= 128;
+  if (t <= 2 * CUS) return !most || batch == 1 || N >= 1024;
+  if (most) return false;
+  if (t <= 4 * CUS) return true;
+  const int64_t rounds = (t + 4 * CUS - 1) / (4 * CUS);
+  return d->a_fmt == OP_BF16 && K >= 4096 && t * 20 >= rounds * (4 * CUS * 17);
 }
 
 int skinny_gemm(const vh_gemm_desc* d, vh_stream_t stream) {

@@ -59,6 +59,7 @@ class GemmDesc(ctypes.Structure):
 
 
 FAMILY_STAGED, FAMILY_DIRECT_FP8, FAMILY_DIRECT_BF16, FAMILY_MXI8, FAMILY_SKINNY = 1, 2, 3, 4, 5
+TILE_SKINNY = 70  # the few-row kernel, whatever the rule of vh_gemm says
 
 #: When set to a list, every ``vh_gemm`` launch appends ``(family, tile,
 #: splits, M, N, K)`` of the kernel it runs (``vh_gemm_plan``), so tests can
@@ -116,7 +117,7 @@ def _bias_operand(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     return bias.contiguous()
 
 
-def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out_dtype, bias=None, alpha=None) -> torch.Tensor:
+def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out_dtype, bias=None, alpha=None, tile_hint: int = 0) -> torch.Tensor:
     """``a[..., M, K] . b[..., N, K]^T`` (bf16 operands, fp32 accumulation),
     ``* alpha + bias`` in fp32, one rounding to ``out_dtype``."""
     if a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
@@ -130,7 +131,7 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out_dtype, bias=None, alpha=None
         K = a.shape[-1]
     if b.dim() == 2 and a.dim() > 2:  # one GEMM over all leading dims
         lead = a.shape[:-1]
-        return gemm_bf16(a.reshape(-1, K), b, out_dtype, bias, alpha).view(*lead, b.shape[0])
+        return gemm_bf16(a.reshape(-1, K), b, out_dtype, bias, alpha, tile_hint).view(*lead, b.shape[0])
     batch_shape = torch.broadcast_shapes(a.shape[:-2], b.shape[:-2]) if a.dim() > 2 or b.dim() > 2 else ()
     M, N = a.shape[-2], b.shape[-2]
     a3 = a.expand(*batch_shape, M, K).reshape(-1, M, K).contiguous() if a.dim() > 2 else a.contiguous()
@@ -152,6 +153,7 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out_dtype, bias=None, alpha=None
     d.batch_stride_a = M * K * 2 if a.dim() > 2 else 0
     d.batch_stride_b = N * K * 2 if bb.dim() > 2 else 0
     d.batch_stride_c = M * N
+    d.tile_hint = tile_hint
     d.epi = _epilogue(EPI_PLAIN, out_dtype, alpha, bias)
     run(d, a.device)
     return out
