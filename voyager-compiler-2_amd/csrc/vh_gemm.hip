@@ -2516,24 +2516,26 @@ int staged_tile(int c) {
 // 17.4 / 23.8 / 25.9 (bf16 39.1 / 54.7 / 55.4 against 27.2 / 40.4 / 45.3);
 // (4096, 14336) at M = 513 / 1111 / 2048 52.9 / 82.6 / 106.8 against 43.7 /
 // 68.7 / 106.6 (bf16, M = 513 / 1111, 94.8 / 150 against 76.5 / 128).
-// Below K = 4096 a tile's own time falls only to f, its launch, fill and
-// store, so short products want fewer, larger tiles (f fitted at K = 256 ..
-// 2048, N = 512 .. 14336, M = 65 .. 8192): with c0 scaled by K alone, as
-// before, the mean over those 528 sizes was 1.8% above the best tile (fp8;
-// bf16 1.7%) and up to 47%, now 0.2% (0.6%) and 13% (19%), one bf16 size of
-// K = 256 apart (M = 8192, N = 1024: 42%).  fp8 at K = 512, M = 4096, N = 2816
-// / 14336 23.6 / 78.8 -> 16.0 / 66.8 us.
+// Below K = 4096 both fall only to f and e, a tile's launch, fill and store, so
+// short products want fewer, larger tiles (f and e fitted at K = 256 .. 3072,
+// N = 512 .. 28672, M = 65 .. 8192): with c0 and c1 scaled by K alone the mean
+// over those sizes (995 of each type) was 1.1% above the best tile (fp8; bf16
+// 1.5%) and up to 47%, now 0.2% (0.8%) and 14% (32%), one bf16 size of K = 256
+// apart (M = 8192, N = 1024: 42%).  fp8 at K = 512, M = 4096, N = 2816 / 14336
+// 23.6 / 78.8 -> 16.0 / 66.8 us.
 struct DlTile {
   int tile, bm, bn;
-  float f, c0, c1;
+  float f, c0, e, c1;
 };
-constexpr DlTile DL_FP8[] = {{37, 64, 128, 3.7f, 10.0f, 1.8f},   {33, 128, 128, 5.3f, 12.4f, 5.0f},
-                             {25, 128, 192, 6.9f, 15.8f, 8.1f},  {31, 256, 128, 8.1f, 18.8f, 10.8f},
-                             {26, 256, 160, 9.4f, 23.2f, 12.6f}, {44, 256, 224, 10.1f, 41.0f, 11.2f},
-                             {41, 256, 256, 8.8f, 42.1f, 15.6f}};
-constexpr DlTile DL_BF16[] = {{35, 128, 64, 3.2f, 17.2f, 3.4f},   {33, 128, 128, 4.4f, 21.2f, 10.3f},
-                              {25, 128, 192, 6.4f, 27.8f, 15.9f}, {31, 256, 128, 7.2f, 33.1f, 21.6f},
-                              {26, 256, 160, 8.1f, 40.0f, 24.6f}, {41, 256, 256, 5.9f, 85.0f, 23.2f}};
+constexpr DlTile DL_FP8[] = {
+    {37, 64, 128, 3.9f, 10.0f, 0.0f, 1.8f},   {33, 128, 128, 5.5f, 12.4f, 0.0f, 5.0f},
+    {25, 128, 192, 6.9f, 15.8f, 0.0f, 8.1f},  {31, 256, 128, 7.9f, 18.8f, 0.4f, 10.8f},
+    {26, 256, 160, 9.3f, 23.2f, 0.4f, 12.6f}, {44, 256, 224, 9.9f, 41.0f, 2.4f, 11.2f},
+    {41, 256, 256, 8.6f, 42.1f, 3.1f, 15.6f}};
+constexpr DlTile DL_BF16[] = {
+    {35, 128, 64, 3.5f, 17.2f, 0.0f, 3.4f},   {33, 128, 128, 4.8f, 21.2f, 0.0f, 10.3f},
+    {25, 128, 192, 6.1f, 27.8f, 0.3f, 15.9f}, {31, 256, 128, 6.6f, 33.1f, 0.9f, 21.6f},
+    {26, 256, 160, 7.5f, 40.0f, 1.1f, 24.6f}, {41, 256, 256, 5.0f, 85.0f, 5.7f, 23.2f}};
 
 template <int NT>
 int dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t K, int64_t batch) {
@@ -2542,7 +2544,8 @@ int dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t K, int64_t batc
   float least = 0.0f;
   for (int i = 0; i < NT; ++i) {
     const int64_t n = ((M + t[i].bm - 1) / t[i].bm) * ((N + t[i].bn - 1) / t[i].bn) * batch;
-    const float us = (float)((n + 255) / 256) * (t[i].f + k * (t[i].c0 - t[i].f)) + (float)n / 256.0f * k * t[i].c1;
+    const float us = (float)((n + 255) / 256) * (t[i].f + k * (t[i].c0 - t[i].f)) +
+                     (float)n / 256.0f * (t[i].e + k * (t[i].c1 - t[i].e));
     if (i == 0 || us < least) best = t[i].tile, least = us;
   }
   return best;

@@ -478,9 +478,9 @@ def mx8_f16_plan(M: int, N: int, K: int) -> Tuple[int, int]:
     round's tiles cost each other, fitted at K = 4096 (M = 513 / 800 / 1111 /
     2048 at K = N = 4096: 29.2 / 34.6 / 44.3 / 67 us, where a choice by rows
     took 42.7 / 41.3 / 48.3 / 67; (4096, 14336): 83.6 / 104 / 143 / 220
-    against 101 / 126 / 163 / 232).  Below K = 4096 the own time falls to the
-    fill and store, as in the other two (K = 256, M = 2500, N = 14336: 59.9 ->
-    46.0 us)."""
+    against 101 / 126 / 163 / 232).  Below K = 4096 both fall to the fill and
+    store, as in the other two (K = 256, M = 2500, N = 14336: 59.9 -> 46.0
+    us)."""
     t64 = -(-M // 64) * -(-N // 64)
     if t64 <= 256:
         return 4, (2 if t64 <= 128 and K % (2 * 512) == 0 else 1)
@@ -489,14 +489,15 @@ def mx8_f16_plan(M: int, N: int, K: int) -> Tuple[int, int]:
 
     def estimate(t):
         n = -(-M // t[1]) * -(-N // t[2])
-        return -(-n // 256) * (t[3] + k * (t[4] - t[3])) + n / 256 * k * t[5]
+        return -(-n // 256) * (t[3] + k * (t[4] - t[3])) + n / 256 * (t[5] + k * (t[6] - t[5]))
 
     return min(_MX8_F16_TILES, key=estimate)[0], 1
 
 
-# (tile, rows, columns, us of a tile at K = 0 and K = 4096, us a full round adds at K = 4096)
-_MX8_F16_TILES = ((1, 64, 128, 3.8, 18.1, 4.1), (0, 128, 128, 5.8, 21.2, 13.3), (5, 128, 192, 8.4, 26.6, 22.0),
-                  (3, 256, 128, 9.0, 32.2, 27.5), (6, 256, 160, 11.6, 40.5, 33.0), (7, 256, 256, 8.3, 81.4, 26.9))
+# (tile, rows, columns, us of a tile at K = 0 and K = 4096, us a full round adds at K = 0 and K = 4096)
+_MX8_F16_TILES = ((1, 64, 128, 3.9, 18.1, 0.0, 4.1), (0, 128, 128, 6.0, 21.2, 0.0, 13.3),
+                  (5, 128, 192, 8.2, 26.6, 0.0, 22.0), (3, 256, 128, 8.7, 32.2, 0.0, 27.5),
+                  (6, 256, 160, 11.3, 40.5, 0.0, 33.0), (7, 256, 256, 7.0, 81.4, 6.1, 26.9))
 
 
 def linear_mx8_f16(x16: torch.Tensor, ex: torch.Tensor, weight: MX8F16Weight, out_dtype=torch.bfloat16, bias=None,
