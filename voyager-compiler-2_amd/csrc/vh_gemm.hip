@@ -430,19 +430,23 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, f32x16 (&acc)[TM][
 }
 
 // Block tile id -> (m0, n0).  Blocks are dealt to the 8 XCDs round robin;
-// tile ids are renumbered so that each XCD gets a contiguous range of them
-// (the first ntiles % 8 XCDs one more), and groups of GM tile-rows are
-// walked column by column so an XCD's blocks share operand panels in its L2
-// (group_rows picks GM).  Without the renumbering, as counts that are no
-// multiple of 8 ran before, 225 tiles of 128 x 192 (bf16, M = 300, K = 4096,
-// N = 14336) take 56.7 us against 44.0.
+// tile ids are renumbered so that each XCD gets a contiguous range of them,
+// and groups of GM tile-rows are walked column by column so an XCD's blocks
+// share operand panels in its L2 (group_rows picks GM).  RAGGED: also where
+// the count is no multiple of 8 (the first ntiles % 8 XCDs get one more): 225
+// tiles of 128 x 192 (bf16, M = 300, K = 4096, N = 14336) take 44.0 us, 56.7
+// without; over 3269 such grids of the direct-to-LDS tiles it takes 2 (bf16)
+// to 5% off (fp8; 13% from three rounds on) and leaves one row tile as it was.
+// The MX-int8 kernels' grids of K splits lose by it (M = 513, K = 1536, N =
+// 2816: 22.7 us, 25.3 with; 1% over 184 grids).
+template <bool RAGGED = false>
 __device__ __forceinline__ void tile_origin(int64_t M, int64_t N, int BM, int BN, int GM, int64_t& m0, int64_t& n0) {
   const int64_t tiles_m = (M + BM - 1) / BM;
   const int64_t tiles_n = (N + BN - 1) / BN;
   const int64_t ntiles = tiles_m * tiles_n;
   int64_t pid = blockIdx.x;
   const int64_t xcd = pid & 7, rest = ntiles & 7;
-  pid = xcd * (ntiles >> 3) + (xcd < rest ? xcd : rest) + (pid >> 3);
+  if (RAGGED || rest == 0) pid = xcd * (ntiles >> 3) + (xcd < rest ? xcd : rest) + (pid >> 3);
   const int64_t group = pid / (GM * tiles_n);
   const int64_t first_m = group * GM;
   const int64_t gsize = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
@@ -1157,7 +1161,7 @@ __global__ void __launch_bounds__(WM * WN * 64, f8dl_wpe(WM * WN))
   const int wm = wave / WN, wn = wave % WN;
 
   int64_t m0, n0;
-  tile_origin(g.M, g.N, BM, BN, g.group_m, m0, n0);
+  tile_origin<true>(g.M, g.N, BM, BN, g.group_m, m0, n0);
   const int64_t bat = blockIdx.y;
   g.A += bat * g.sa;
   g.B += bat * g.sb;
