@@ -55,8 +55,9 @@ FEW_ROWS = {
     gemm.OP_FP8: {True: [(1, 4096, 64, 1), (64, 4096, 512, 1), (16, 8192, 512, 1), (32, 14336, 4096, 1)],
                   False: [(32, 8192, 512, 1), (1, 14336, 1024, 1), (64, 14336, 4096, 1), (1, 20480, 4096, 1),
                           (16, 32768, 14336, 1)]},
-    gemm.OP_MXI8: {True: [(16, 4096, 128, 1), (32, 14336, 256, 1), (64, 4096, 4096, 1), (1, 65536, 512, 1)],
-                   False: [(16, 4096, 64, 1), (17, 4096, 128, 1), (64, 4112, 4096, 1), (1, 28672, 256, 1)]},
+    gemm.OP_MXI8: {True: [(16, 4096, 128, 1), (32, 14336, 256, 1), (64, 4096, 4096, 1), (1, 65536, 256, 1),
+                          (1, 28672, 1024, 1)],
+                   False: [(16, 4096, 64, 1), (17, 4096, 128, 1), (64, 4112, 4096, 1), (1, 28672, 576, 1)]},
 }
 
 
@@ -66,3 +67,10 @@ def test_few_rows(fmt, few, M, N, K, batch):
     assert (_plan(fmt, M, N, K, batch)[0] == gemm.FAMILY_SKINNY) == few
     if M <= 64:
         assert _plan(fmt, M, N, K, batch, gemm.TILE_SKINNY)[0] == gemm.FAMILY_SKINNY
+
+
+@pytest.mark.parametrize("fmt", [gemm.OP_BF16, gemm.OP_FP8, gemm.OP_MXI8])
+@pytest.mark.parametrize("M,N", [(0, 64), (4, 0), (0, 0)])
+def test_empty_products(fmt, M, N):
+    _plan(fmt, M, N, 64)
+    _plan(fmt, M, N, 64, 3)

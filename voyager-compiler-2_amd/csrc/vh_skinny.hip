@@ -597,13 +597,15 @@ bool skinny_taken(const vh_gemm_desc* d) {
   // .. 256) the choice is 0.6% above the faster kernel on average; any K and,
   // to 32 rows, any grid, as before, 9.7%.
   if (d->tile_hint == VH_GEMM_TILE_SKINNY) return skinny_fits(d);
-  if (d->tile_hint != 0 || d->split_k != 0 || !skinny_fits(d)) return false;
+  if (d->tile_hint != 0 || d->split_k != 0 || d->N <= 0 || !skinny_fits(d)) return false;
   const int64_t batch = d->batch < 1 ? 1 : d->batch, K = d->K, N = d->N;
   const int64_t t = (N + 15) / 16 * batch;  // tiles of 16 weight rows
   const bool many = d->M > 16, most = d->M > 32;
+  const int64_t rounds = (t + 4 * CUS - 1) / (4 * CUS);  // at NT = 4
+  const int64_t fill = t * 20 / (rounds * 4 * CUS);      // of them, in twentieths
   if (d->a_fmt == OP_MXI8) {
     if (most && (N > 4096 || K > 4096)) return false;
-    return K >= (t > 4 * CUS ? 512 : many ? 256 : 128);
+    return K >= (rounds > 1 && fill < 18 ? 1024 : many || rounds > 1 ? 256 : 128);
   }
   if (K < 2048) {
     if (t <= CUS) return batch == 1 || t <= (most ? 64 : many ? 128 : CUS);
@@ -612,9 +614,7 @@ bool skinny_taken(const vh_gemm_desc* d) {
   if (t <= CUS) return !most || batch == 1 || N >= 512 || t <= 128;
   if (t <= 2 * CUS) return !most || batch == 1 || N >= 1024;
   if (most) return false;
-  if (t <= 4 * CUS) return true;
-  const int64_t rounds = (t + 4 * CUS - 1) / (4 * CUS);
-  return d->a_fmt == OP_BF16 && K >= 4096 && t * 20 >= rounds * (4 * CUS * 17);
+  return rounds == 1 || (d->a_fmt == OP_BF16 && K >= 4096 && fill >= 17);
 }
 
 int skinny_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
