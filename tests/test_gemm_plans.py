@@ -32,7 +32,9 @@ def _plan(fmt, M, N, K, batch=1, hint=0):
     (gemm.OP_BF16, 1500, 8960, 512, 41),
     # from K = 4096 on
     (gemm.OP_FP8, 513, 4096, 4096, 33), (gemm.OP_FP8, 1111, 4096, 14336, 25), (gemm.OP_FP8, 2048, 14336, 4096, 44),
-    (gemm.OP_BF16, 300, 14336, 4096, 25), (gemm.OP_BF16, 2048, 4096, 14336, 31)])
+    (gemm.OP_BF16, 300, 14336, 4096, 25), (gemm.OP_BF16, 2048, 4096, 14336, 31),
+    # many tiles of 256 x 256 are not the fastest
+    (gemm.OP_BF16, 2048, 14336, 4096, 26), (gemm.OP_BF16, 3000, 8192, 3072, 31), (gemm.OP_BF16, 4096, 8960, 14336, 26)])
 def test_direct_tiles(fmt, M, N, K, tile):
     family = gemm.FAMILY_DIRECT_FP8 if fmt == gemm.OP_FP8 else gemm.FAMILY_DIRECT_BF16
     assert _plan(fmt, M, N, K) == (family, tile)

@@ -49,7 +49,7 @@ class _Plans:
 CFG2 = [
     ((4096, 4096), 31, 31),
     ((4096, 1024), 37, 35),
-    ((4096, 14336), 44, 41),
+    ((4096, 14336), 44, 26),
     ((14336, 4096), 31, 31),
 ]
 
@@ -116,10 +116,12 @@ def test_cfg4_posit8_gemm_full_size():
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
-    (2048, 14336, 4096, 41),   # >= 384 tiles of 256 x 256
-    (2048, 4096, 4096, 31),    # >= 224 tiles of 256 x 128
-    (1024, 3584, 2048, 33),    # >= 224 tiles of 128 x 128
-    (256, 4096, 4096, 35),     # fewer: 128 x 64
+    (2048, 14336, 4096, 26),   # 256 x 160: three rounds of 256 CUs
+    (1024, 14336, 256, 41),    # 256 x 256: one round, short K
+    (300, 14336, 4096, 25),    # 128 x 192
+    (2048, 4096, 4096, 31),    # 256 x 128
+    (1024, 3584, 2048, 33),    # 128 x 128
+    (256, 4096, 4096, 35),     # 128 x 64
 ])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_bf16_direct_tiles(M, N, K, tile, out_dtype):

@@ -2524,7 +2524,7 @@ int staged_tile(int c) {
 // short products want fewer, larger tiles (f and e fitted at K = 256 .. 3072,
 // N = 512 .. 28672, M = 65 .. 8192): with c0 and c1 scaled by K alone the mean
 // over those sizes (995 of each type) was 1.1% above the best tile (fp8; bf16
-// 1.5%) and up to 47%, now 0.2% (0.8%) and 14% (32%), one bf16 size of K = 256
+// 1.5%) and up to 47%, now 0.2% (0.4%) and 14% (18%), one bf16 size of K = 256
 // apart (M = 8192, N = 1024: 42%).  fp8 at K = 512, M = 4096, N = 2816 / 14336
 // 23.6 / 78.8 -> 16.0 / 66.8 us.
 struct DlTile {
@@ -2541,18 +2541,21 @@ constexpr DlTile DL_BF16[] = {
     {25, 128, 192, 6.1f, 27.8f, 0.3f, 15.9f}, {31, 256, 128, 6.6f, 33.1f, 0.9f, 21.6f},
     {26, 256, 160, 7.5f, 40.0f, 1.1f, 24.6f}, {41, 256, 256, 5.0f, 85.0f, 5.7f, 23.2f}};
 
+float dl_us(const DlTile& t, int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const float k = K < 4096 ? (float)K / 4096.0f : 1.0f, more = K > 4096 ? (float)K / 4096.0f : 1.0f;
+  const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch;
+  return more * ((float)((n + 255) / 256) * (t.f + k * (t.c0 - t.f)) + (float)n / 256.0f * (t.e + k * (t.c1 - t.e)));
+}
+
 template <int NT>
-int dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t K, int64_t batch) {
-  const float k = K < 4096 ? (float)K / 4096.0f : 1.0f;  // (from there on every term grows alike)
-  int best = t[0].tile;
+const DlTile& dl_tile(const DlTile (&t)[NT], int64_t M, int64_t N, int64_t K, int64_t batch) {
+  int best = 0;
   float least = 0.0f;
   for (int i = 0; i < NT; ++i) {
-    const int64_t n = ((M + t[i].bm - 1) / t[i].bm) * ((N + t[i].bn - 1) / t[i].bn) * batch;
-    const float us = (float)((n + 255) / 256) * (t[i].f + k * (t[i].c0 - t[i].f)) +
-                     (float)n / 256.0f * (t[i].e + k * (t[i].c1 - t[i].e));
-    if (i == 0 || us < least) best = t[i].tile, least = us;
+    const float us = dl_us(t[i], M, N, K, batch);
+    if (i == 0 || us < least) best = i, least = us;
   }
-  return best;
+  return t[best];
 }
 
 // The one dispatch rule of vh_gemm: which kernel and tile a descriptor runs
@@ -2584,17 +2587,12 @@ Plan plan_gemm(const vh_gemm_desc* d) {
   // validated a multiple of 16 below, where the descriptor is checked).
   const bool chunks_ok = d->lda % 16 == 0 && d->ldb % 16 == 0 && d->K % (fp8 ? 16 : 8) == 0;
   if (fp8 && dl_ok && chunks_ok) {
-    const int c = d->tile_hint ? d->tile_hint : dl_tile(DL_FP8, d->M, d->N, d->K, batch);
+    const int c = d->tile_hint ? d->tile_hint : dl_tile(DL_FP8, d->M, d->N, d->K, batch).tile;
     if (is_direct_fp8_tile(c)) return {FAM_DIRECT_FP8, c, 1};
   }
   if (fp8) return {FAM_STAGED, staged, 1};
   if (d->a_fmt == OP_BF16 && d->b_fmt == OP_BF16 && dl_ok && chunks_ok && (d->tile_hint == 0 || d->tile_hint >= 20)) {
-    // From 384 tiles of 256 x 256 those stay: the estimate would take 256 x
-    // 160 there, 192-200 us against 204-214 at M = 1800-2048, K = 4096, N =
-    // 14336 alone, but even within a run of other kernels.
-    const int c = d->tile_hint ? d->tile_hint
-                  : tiles(256, 256) >= 384 ? 41
-                                           : dl_tile(DL_BF16, d->M, d->N, d->K, batch);
+    const int c = d->tile_hint ? d->tile_hint : dl_tile(DL_BF16, d->M, d->N, d->K, batch).tile;
     if (is_direct_bf16_tile(c)) return {FAM_DIRECT_BF16, c, 1};
   }
   if (d->a_fmt == OP_MXI8 && d->b_fmt == OP_MXI8) {
