@@ -1,9 +1,12 @@
 """The kernels and tiles the GEMM dispatch picks, evaluated on the host: the
 sizes its rules were measured at, either side of each line they draw."""
 
+import ctypes
+
 import pytest
 
 from voyager_amd import gemm
+from voyager_amd._lib import load
 
 
 def _plan(fmt, M, N, K, batch=1, hint=0):
@@ -76,3 +79,15 @@ def test_few_rows(fmt, few, M, N, K, batch):
 def test_empty_products(fmt, M, N):
     _plan(fmt, M, N, 64)
     _plan(fmt, M, N, 64, 3)
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 1536, 8960), (256, 1536, 8960), (201, 1280, 4096), (300, 3072, 4096),
+                                   (512, 2816, 4096), (64, 8960, 512), (400, 4608, 2048), (256, 4096, 4096)])
+def test_nf4_splits_fill_one_round(M, N, K):
+    """As many K ranges as one round of 256 workgroups takes, and no more."""
+    sp = ctypes.c_int32(0)
+    assert load().vh_gemm_nf4_bf16_plan(M, N, K, ctypes.byref(sp)) == 0
+    tiles, blocks = -(-M // 256) * -(-N // 64), K // 64
+    most = max(1, min(256 // tiles, blocks // 4))
+    assert tiles * sp.value <= 256
+    assert sp.value == -(-blocks // -(-blocks // most))  # ranges of whole blocks
