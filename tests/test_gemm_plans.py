@@ -91,3 +91,15 @@ def test_nf4_splits_fill_one_round(M, N, K):
     most = max(1, min(256 // tiles, blocks // 4))
     assert tiles * sp.value <= 256
     assert sp.value == -(-blocks // -(-blocks // most))  # ranges of whole blocks
+
+
+# (M, N, K): two passes, or the weight decoded in the GEMM
+TWO_PASS = {True: [(512, 4096, 1024), (511, 4096, 4096), (700, 4096, 4096), (400, 14336, 4096), (1000, 1024, 4096),
+                   (1025, 512, 14336), (300, 8960, 2048)],
+            False: [(17, 14336, 4096), (256, 4096, 14336), (300, 4096, 4096), (300, 14336, 4096), (511, 4096, 14336),
+                    (512, 1024, 4096), (700, 1024, 14336), (300, 8192, 1024), (300, 14336, 512), (300, 1024, 64)]}
+
+
+@pytest.mark.parametrize("two,M,N,K", [(t,) + c for t, cs in TWO_PASS.items() for c in cs])
+def test_nf4_two_pass(two, M, N, K):
+    assert gemm.nf4_two_pass_pays(M, N, K) == two

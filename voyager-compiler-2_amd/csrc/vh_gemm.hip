@@ -2916,6 +2916,23 @@ extern "C" int vh_gemm_nf4_bf16_plan(int64_t M, int64_t N, int64_t K, int32_t* s
   return VH_OK;
 }
 
+extern "C" int vh_gemm_nf4_two_pass(int64_t M, int64_t N, int64_t K) {
+  // One row tile covers up to 256 rows; past four of them the bf16 GEMM's
+  // twice as high rate always wins.  Between, both forms by estimate, fitted in
+  // us to whole linears of M = 257 .. 1024, K >= 1024, N = 256 .. 32768 (the
+  // table in voyager_amd/gemm.py): the choice is 0.7% above the better form on
+  // average over 1311 of them; by rows and columns alone, as before, 6.1%.
+  if (M <= 256 || M > 1024 || N < 1 || K < 64) return M > 256;
+  const Nf4bPlan p = nf4b_plan(M, N, K, 0);
+  const float h = (float)p.bm / 64.0f, groups = (float)p.tiles * (float)p.splits;
+  const float rounds = (float)((p.tiles * p.splits + 255) / 256);
+  const float mn = (float)M * (float)N * 1e-6f, nk = (float)N * (float)K * 1e-6f;
+  const float one = 7.9f + rounds * (p.kcs * (0.202f + 0.075f * h) + 2.38f * h) + groups / 256.0f * p.kcs * 0.047f * h +
+                    (p.splits > 1 ? 1.97f * p.splits * mn : 0.0f);
+  const float two = 11.3f + 0.514f * nk + 1.07f * dl_us(dl_tile(DL_BF16, M, N, K, 1), M, N, K, 1);
+  return one > two;
+}
+
 extern "C" int vh_gemm_nf4_bf16(const uint16_t* x, int64_t M, const uint8_t* w_packed, const uint8_t* w_scale,
                                 const vh_format* w_scale_fmt, const int8_t* levels16, int64_t N, int64_t K,
                                 const vh_epilogue* epi, void* y, int64_t ldy, int32_t splits, float* part,

@@ -670,18 +670,18 @@ def linear_nf4_prefill(x: torch.Tensor, weight: NF4Weight, index_table: torch.Te
                        splits: int = 0, two_pass: Optional[bool] = None) -> torch.Tensor:
     """MXNF4 ``linear_mx`` at any M on the GEMV's baked weight: both operands
     decoded to the reference's ``bf16(level * scale)`` and multiplied on the
-    bf16 MFMA with float32 accumulation.  Up to 256 rows (and by few columns,
-    ``nf4_two_pass_pays``) the activation is quantized straight to those
-    values and the weight decoded in the GEMM (``vh_gemm_nf4_bf16``); else,
-    or at a given ``tile`` / ``splits`` / ``two_pass``, its ``quantize_mx``
-    goes to index and scale bytes for ``gemm_nf4_packed``."""
+    bf16 MFMA with float32 accumulation.  Where ``vh_gemm_nf4_bf16`` takes it
+    (``_nf4_route``) the activation is quantized straight to those values and
+    the weight decoded in the GEMM; else, or at a given ``tile`` / ``splits``
+    / ``two_pass``, its ``quantize_mx`` goes to index and scale bytes for
+    ``gemm_nf4_packed``."""
     from . import packed as _packed
 
     M, K = x.shape
     if K != weight.K:
         raise RuntimeError("linear_nf4_prefill: contraction mismatch")
     x = x.contiguous()
-    if two_pass is None and tile == 0 and splits == 0 and _nf4_bf16_pays(M, weight):
+    if two_pass is None and tile == 0 and splits == 0 and _nf4_route(M, weight) == "bf16":
         ec, sc = formats.classify(index_table), formats.classify(scale_qmap)
         if _nf4_index_quantize(x, ec, sc) and x.data_ptr() % 16 == 0:
             return gemm_nf4_bf16(nf4_quantize_bf16(x, weight, ec, sc), weight, out_dtype, bias, alpha)
@@ -689,11 +689,22 @@ def linear_nf4_prefill(x: torch.Tensor, weight: NF4Weight, index_table: torch.Te
     return gemm_nf4_packed(px, weight, out_dtype, bias, alpha, tile, splits, two_pass)
 
 
-def _nf4_bf16_pays(M: int, weight: NF4Weight) -> bool:
-    """Whether ``vh_gemm_nf4_bf16`` takes the prefill: where
-    ``nf4_two_pass_pays`` does not, and the weight lies as its loads need."""
-    return (M >= 1 and not nf4_two_pass_pays(M, weight.N, weight.K) and weight.K <= 1 << 20
-            and weight.packed.data_ptr() % 16 == 0 and weight.scale.data_ptr() % 16 == 0)
+def _nf4_route(M: int, weight: NF4Weight) -> str:
+    """The kernels of an MXNF4 prefill: "two" (``nf4_two_pass_pays``), "bf16"
+    (``vh_gemm_nf4_bf16``) or "fused" (``vh_gemm_nf4``): where the weight does
+    not lie as the second's loads need, and for short K, whose few blocks do
+    not pay for its setup (M = 256, K = 64: 17.6 us against 10.7; K = 512, N =
+    14336, M = 300: 29.4 against 23.8, K = 1024 37.4 against 36.7)."""
+    N, K = weight.N, weight.K
+    if nf4_two_pass_pays(M, N, K):
+        return "two"
+    fits = K <= 1 << 20 and weight.packed.data_ptr() % 16 == 0 and weight.scale.data_ptr() % 16 == 0
+    return "bf16" if M >= 1 and fits and not _nf4_short(M, N, K) else "fused"
+
+
+def _nf4_short(M: int, N: int, K: int) -> bool:
+    """Too few blocks of K for ``vh_gemm_nf4_bf16`` and the two passes alike."""
+    return M < 512 and (K <= 128 and (M >= 64 or N > 16384) or K < 1024 and N > 8192 and M > 256)
 
 
 def nf4_quantize_bf16(x: torch.Tensor, weight: NF4Weight, ec, sc) -> torch.Tensor:
@@ -733,37 +744,40 @@ def nf4_two_pass_pays(M: int, N: int, K: int) -> bool:
     """Whether the prefill runs as two passes (both operands decoded once,
     then the bf16 GEMM) rather than on ``vh_gemm_nf4_bf16``, which decodes a
     weight block once per 256 rows and multiplies at half the bf16 GEMM's
-    rate.  Measured on MI355X (``vh_gemm_nf4_bf16`` with the activation's
-    decode / two-pass, us): (K, N) = (4096, 4096) at M = 256: 29.6 / 32.5,
-    300: 31.2 / 32.9, 512: 39.1 / 34.2; (4096, 14336): 57.0 / 61.8, 80.1 /
-    74.1, 103 / 77.9; (14336, 4096): 55.4 / 87.8, 68.0 / 91.5, 99.9 / 102;
-    (4096, 1024): 25.8 / 26.8, 21.8 / 30.5, 24.5 / 30.5.  So up to 256 rows
-    the one tile of rows decides, and above them only columns too few to
-    fill the chip do.  The two-pass form holds the decoded weight (2 bytes
-    per element) for the call."""
-    return M >= NF4_TWO_PASS_MIN_M or (M > 256 and N > 2048)
+    rate.  Measured on MI355X, whole linears (``vh_gemm_nf4_bf16`` / two-pass,
+    us), (K, N) at M = 256, 300, 400, 511, 700, 1000:
 
+    (2048, 4096)   28.4 / 28.2  26.9 / 29.4  30.8 / 27.9  33.4 / 29.2  40.0 / 33.6  44.4 / 35.4
+    (4096, 1024)   28.2 / 32.6  25.4 / 36.4  26.5 / 37.3  28.4 / 35.9  33.6 / 36.9  36.1 / 37.2
+    (4096, 4096)   30.9 / 36.2  33.5 / 38.2  39.6 / 40.0  44.0 / 42.0  62.8 / 48.1  68.5 / 56.0
+    (4096, 14336)  61.4 / 74.8  85.8 / 92.4   102 / 98.0   115 / 102    163 / 137    219 / 157
+    (14336, 4096)  58.9 / 107   72.5 / 113   89.4 / 121    105 / 131    167 / 155    186 / 177
 
-#: Rows from which the two-pass MXNF4 prefill is taken at every N.
-NF4_TWO_PASS_MIN_M = 512
+    Up to 256 rows the one tile of rows decides.  Above, a row costs the first
+    more and the weight's decode, which grows with K and N, is saved once;
+    both in rounds of the CUs, so ``vh_gemm_nf4_two_pass`` compares the two by
+    estimate.  The two-pass form holds the decoded weight (2 bytes per
+    element) for the call."""
+    return not _nf4_short(M, N, K) and bool(load().vh_gemm_nf4_two_pass(M, N, K))
 
 
 def gemm_nf4_packed(px, weight: NF4Weight, out_dtype=torch.bfloat16, bias=None, alpha=None, tile: int = 0,
                     splits: int = 0, two_pass: Optional[bool] = None) -> torch.Tensor:
     """The MXNF4 linear of an activation already packed by
     ``quantize_mx_packed`` (index bytes [M, K] and scale codes [M, K / 64]):
-    with ``two_pass`` (by default where ``nf4_two_pass_pays``) the operands
-    decoded once by ``nf4_decode_bf16`` and multiplied by the bf16 GEMM;
-    without, or at a given tile or split, ``vh_gemm_nf4``, which decodes both
-    while staging; by default below that the activation decoded once and
-    ``vh_gemm_nf4_bf16``.  All give the same products, summed in another
+    with ``two_pass`` the operands decoded once by ``nf4_decode_bf16`` and
+    multiplied by the bf16 GEMM; without, or at a given tile or split,
+    ``vh_gemm_nf4``, which decodes both while staging; by default
+    ``_nf4_route``'s choice of those and ``vh_gemm_nf4_bf16`` on the
+    activation decoded once.  All give the same products, summed in another
     order."""
     M, K = px.codes.shape
     if K != weight.K:
         raise RuntimeError("gemm_nf4_packed: contraction mismatch")
     if two_pass is None:
-        two_pass = nf4_two_pass_pays(M, weight.N, K)
-        if tile == 0 and splits == 0 and _nf4_bf16_pays(M, weight):
+        route = _nf4_route(M, weight)
+        two_pass = route == "two"
+        if tile == 0 and splits == 0 and route == "bf16":
             xo, _ = nf4_decode_bf16(px, weight, decode_w=False)
             return gemm_nf4_bf16(xo, weight, out_dtype, bias, alpha)
     if two_pass:
