@@ -5,7 +5,7 @@ import ctypes
 
 import pytest
 
-from voyager_amd import gemm
+from voyager_amd import gemm, lower
 from voyager_amd._lib import load
 
 
@@ -103,3 +103,11 @@ TWO_PASS = {True: [(512, 4096, 1024), (511, 4096, 4096), (700, 4096, 4096), (400
 @pytest.mark.parametrize("two,M,N,K", [(t,) + c for t, cs in TWO_PASS.items() for c in cs])
 def test_nf4_two_pass(two, M, N, K):
     assert gemm.nf4_two_pass_pays(M, N, K) == two
+
+
+@pytest.mark.parametrize("N,full", [(64, True), (16384, True), (16400, False), (20480, False), (28672, False),
+                                    (32768, True), (32832, False), (65536, True), (128256, True)])
+def test_one_launch_rounds(N, full):
+    """The E4M3 linear that quantizes its rows in the launch: not where a
+    round of its workgroups would be mostly empty."""
+    assert lower._full_rounds(N) == full
