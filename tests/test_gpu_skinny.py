@@ -149,3 +149,13 @@ def test_rows8_nan_and_infinity():
         two = gemm.linear_fp8(packed.quantize_packed(x, sx, tabf), wq, sx)
         one = lower.lowered_fp8_linear(x, sx, tabf, wq, sx)
         assert torch.equal(one.nan_to_num(12345.0), two.nan_to_num(12345.0)) and one.isnan().any()
+
+
+@pytest.mark.parametrize("rows", [4, 16])
+def test_fp8_scale_of_more_dims_is_refused(rows):
+    """A scale with more dimensions than the activation's rows does not
+    broadcast to them, however many rows there are."""
+    x, w = torch.zeros(rows, 64).bfloat16().cuda(), torch.zeros(32, 64, dtype=torch.uint8, device="cuda")
+    scale = torch.ones(1, 1, 1, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(ValueError, match="more dims"):
+        lower.lowered_fp8_linear(x, scale, formats.quantization_map("fp8_e4m3"), w, scale.reshape(()))

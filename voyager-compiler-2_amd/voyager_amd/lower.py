@@ -322,7 +322,7 @@ def lowered_fp8_linear(x, x_scale, qmap, w_bytes, out_scale):
     on E4M3 bytes (at decode sizes in one launch)."""
     xr = _rows(x)
     if (_one_launch(xr, w_bytes) and (xr.shape[0] <= 4 or xr.shape[1] <= 8192) and _full_rounds(w_bytes.shape[0])
-            and x_scale.dtype == torch.bfloat16 and x_scale.numel() == 1
+            and x_scale.dtype == torch.bfloat16 and x_scale.numel() == 1 and x_scale.dim() <= 2
             and formats.classify(qmap).fmt.flags & FMT_HW_E4M3):
         return gemm.linear_fp8_rows8(xr, x_scale, w_bytes, out_scale).reshape(*x.shape[:-1], w_bytes.shape[0])
     xq = packed.quantize_packed(xr, x_scale, qmap)
