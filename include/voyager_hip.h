@@ -75,6 +75,10 @@ typedef struct vh_format {
 #define VH_ABI_VERSION 2
 
 const char* vh_last_error(void);
+/* The kernel that the calling thread's last vh_quantize_mx, vh_quantize_affine
+ * or vh_dequantize launched, without its template arguments: these choose one
+ * by format, layout, size and alignment.  "" before the first.  For tests. */
+const char* vh_last_kernel(void);
 int vh_abi_version(void);
 
 /* Rebuild a format's 65,536-entry table (bfloat16 bits, entry i for input

@@ -1,8 +1,8 @@
 """The block-scaled quantize and dequantize kernels of one mode and map each
 (``vh_blockfast.h``, ``k_dequantize_blocks``) against the general kernels, bit
-for bit: the same values behind a 16-byte aligned address, which they need, and
-behind one that is not, over every form they take, at edges of blocks, rows and
-workgroups, with zeros, NaN, infinities, subnormal and huge blocks, quotients on
+for bit and with the kernel that ran asserted: the same values behind a 16-byte
+aligned address, which they need, and behind one that is not, over every form
+they take, at edges of blocks, rows and workgroups, with zeros, NaN, infinities, subnormal and huge blocks, quotients on
 rounding midpoints and scales that saturate or flush their map; a case of each
 against the oracle."""
 
@@ -13,6 +13,7 @@ import voyager_amd.library  # noqa: F401  (defines quantized_ops)
 from helpers import assert_same_bits
 from oracle import ops as O
 from oracle import tables as T
+from voyager_amd._lib import load
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +25,10 @@ FORMS = [("int8", 16, 127.0, "pot"), ("fp8_e4m3", 32, 448.0, "pot"), ("fp4_e2m1"
 # rows, columns: over 2**18 elements where the blocks run along a row, so that
 # the one-element-a-lane kernels of small tensors do not take it; partial blocks
 SHAPES = [(65, 4096), (300, 904), (77, 8200), (2, 131080)]
+
+
+def _ran():
+    return load().vh_last_kernel().decode()
 
 
 def _unaligned(t):
@@ -70,6 +75,7 @@ def _quantize(q, x, axis, form, tab, stab, mid):
 @pytest.mark.parametrize("form", FORMS, ids=lambda f: f"{f[0]}-{f[1]}-{f[3]}")
 @pytest.mark.parametrize("axis", [-1, -2])
 def test_same_as_general_kernels(form, axis):
+    """... and back; only aligned tensors take the kernels under test."""
     q = torch.ops.quantized_ops
     tab, stab, mid, entries = _tables(form[0], form[3])
     for rows, cols in SHAPES:
@@ -79,15 +85,23 @@ def test_same_as_general_kernels(form, axis):
             if x.shape[-1] % 8:  # a multiple of eight inside the blocked dimension, which the column form needs
                 x = torch.nn.functional.pad(x, (0, -x.shape[-1] % 8))
         fast = _quantize(q, x, axis, form, tab, stab, mid)
+        assert _ran() == ("k_fast_rows" if axis == -1 else "k_fast_cols"), _ran()
         general = _quantize(q, _unaligned(x), axis, form, tab, stab, mid)
+        # (MX integers along rows have a kernel of their own behind any address)
+        own = axis == -1 and form[0].startswith("int") and form[3] == "pot"
+        assert _ran() == ("k_mx_pot_int_rows8" if own else "k_rows" if axis == -1 else "k_cols"), _ran()
         for a, b, what in zip(fast, general, ("scale", "codes or zero point", "codes")):
             assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"{what} of {list(x.shape)}"
         codes, scale = fast[-1], fast[0]
-        if form[3].startswith("affine"):
-            args = (scale, fast[1], [axis], form[1])
-            one, two = q.dequantize(codes, *args), q.dequantize(_unaligned(codes), *args)
-        else:
-            one, two = (q.dequantize_mx(c, scale, form[1], entries) for c in (codes, _unaligned(codes)))
+
+        def back(c):
+            if form[3].startswith("affine"):
+                return q.dequantize(c, scale, fast[1], [axis], form[1])
+            return q.dequantize_mx(c, scale, form[1], entries)
+
+        one, ran = back(codes), _ran()
+        two = back(_unaligned(codes))
+        assert (ran, _ran()) == ("k_dequantize_blocks", "k_dequantize"), list(x.shape)
         assert torch.equal(one.view(torch.int16), two.view(torch.int16)), f"dequantize of {list(x.shape)}"
 
 
@@ -98,6 +112,7 @@ def test_same_as_oracle(form, axis):
     x = _values(72, 4104, 3)
     tab, stab, mid, _ = _tables(form[0], form[3])
     got = _quantize(q, x, axis, form, tab, stab, mid)
+    assert _ran() == ("k_fast_rows" if axis == -1 else "k_fast_cols"), _ran()
     ctab, cstab, cmid, _ = _tables(form[0], form[3], "cpu")
     exp = _quantize(O, x.cpu(), axis, form, ctab, cstab, cmid)
     for a, b, what in zip(got, exp, ("scale", "codes or zero point", "codes")):
@@ -120,5 +135,8 @@ def test_dequantize_layouts(shape, axis):
     s, z = (torch.randn(*ps, generator=g).bfloat16().cuda() for _ in range(2))
     one = torch.tensor(0.37, device="cuda")
     for args in ((s, z, [axis], 32), (s, None, [axis], 32), (one,), (one.bfloat16(),)):
-        a, b = q.dequantize(x, *args), q.dequantize(_unaligned(x), *args)
+        a, ran = q.dequantize(x, *args), _ran()
+        b = q.dequantize(_unaligned(x), *args)
+        assert _ran() == "k_dequantize"
+        assert ran == ("k_dequantize_blocks" if shape[-1] % 8 == 0 else "k_dequantize"), args[2:]
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), args[2:]

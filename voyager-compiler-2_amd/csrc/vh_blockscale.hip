@@ -502,6 +502,7 @@ bool launch_fast(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t
     const uint32_t threads = (uint32_t)(outer * nblk * g);
     return dispatch_fast(P, [&](auto m, auto k, auto s) {
       constexpr int M = decltype(m)::value, K = decltype(k)::value, S = decltype(s)::value;
+      vh::note_kernel("k_fast_rows");
       const dim3 grid((threads + 255) / 256);
       if (L % block == 0)
         hipLaunchKernelGGL((k_fast_rows<M, K, S, true>), grid, dim3(256), 0, stream, xp, threads, (uint32_t)L,
@@ -520,6 +521,7 @@ bool launch_fast(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t
       hipLaunchKernelGGL(kern, dim3((total + 63) / 64), dim3(256), 0, stream, xp, total, L, inner,
                          make_fast_div((uint32_t)(inner / 8)), make_fast_div((uint32_t)nblk), P, sp, zp, cp);
     };
+    vh::note_kernel("k_fast_cols");
     if (block == 16) go(k_fast_cols<M, K, S, 4>);
     else if (block == 32) go(k_fast_cols<M, K, S, 8>);
     else go(k_fast_cols<M, K, S, 16>);
@@ -545,11 +547,13 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
   if (!steps_lanes && !lanes_ok && launch_fast(x, outer, L, inner, block, P, scale_out, zp_out, codes_out, rows_ok, stream))
     return vh::check_launch(what);
   if (steps_lanes) {
+    vh::note_kernel("k_mx_steps_lanes");
     const int64_t threads = outer * L;
     hipLaunchKernelGGL(k_mx_steps_lanes, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
                        (const uint16_t*)x, outer, L, nblk, (int)block, P.quant_max, P.sfmt, P.fmt, P.scale_t16,
                        P.scale_dtype == VH_F32 ? 1 : 0, scale_out, (uint8_t*)codes_out, P.code_lut);
   } else if (lanes_ok) {
+    vh::note_kernel("k_rows");
     const int g = (int)block;
     const int64_t threads = outer * nblk * g;
     const int64_t blocks = (threads + 255) / 256;
@@ -576,6 +580,7 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
                           P.scale_dtype == VH_BF16 && !P.code_lut && !P.gs && !P.scale_t16 && codes_out &&
                           P.has_fmt && !P.has_sfmt && k0 == K_INT;
     if ((lean && P.mode == MX_POT && k0 == K_INT && !P.has_sfmt) || lean_ref) {
+      vh::note_kernel("k_mx_pot_int_rows8");
       const bool i32 = blocks * 256 < (1ll << 31);
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)x, outer, L, nblk, g,
@@ -589,6 +594,7 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
         else go(k_mx_pot_int_rows8<int64_t, false>);
       }
     } else if (lean && P.mode == MX_SCALED && k0 == K_STEPS && P.has_sfmt && kernel_kind(&P.sfmt) == K_MINI) {
+      vh::note_kernel(P.fmt.nsteps <= 15 ? "k_mx_steps_rows8" : "k_rows");
       if (P.fmt.nsteps <= 15) {
         if (blocks * 256 < (1ll << 31))
           hipLaunchKernelGGL(k_mx_steps_rows8<uint32_t>, dim3((unsigned)blocks), dim3(256), 0, stream,
@@ -603,6 +609,7 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
                            outer, L, nblk, g, P, scale_out, zp_out, codes_out);
       }
     } else {
+      vh::note_kernel("k_rows");
       dispatch_kind(k0, [&](auto kind) {
         constexpr int K = decltype(kind)::value;
         return dispatch_scale(P, [&](auto skind) {
@@ -617,6 +624,7 @@ int launch(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block
     const int64_t threads = outer * nblk * inner;
     const int64_t blocks = (threads + 255) / 256;
     VH_REQUIRE(blocks < (1ll << 31), "%s: tensor too large", what);
+    vh::note_kernel("k_cols");
     dispatch_kind(P.has_fmt ? kernel_kind(&P.fmt) : (int)K_NONE, [&](auto kind) {
       constexpr int K = decltype(kind)::value;
       return dispatch_scale(P, [&](auto skind) {

@@ -21,6 +21,7 @@
 namespace vh {
 
 static thread_local std::string g_error;
+static thread_local const char* g_kernel = "";
 
 void set_error(const char* fmt, ...) {
   char buf[512];
@@ -30,6 +31,8 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
   g_error = buf;
 }
+
+void note_kernel(const char* name) { g_kernel = name; }
 
 int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
@@ -43,6 +46,7 @@ int check_launch(const char* what) {
 }  // namespace vh
 
 extern "C" const char* vh_last_error(void) { return vh::g_error.c_str(); }
+extern "C" const char* vh_last_kernel(void) { return vh::g_kernel; }
 extern "C" int vh_abi_version(void) { return VH_ABI_VERSION; }
 
 // ------------------------------------------------------------ table rebuild
@@ -1415,6 +1419,7 @@ static bool launch_dequantize_blocks(const void* x, int64_t n, const Shape& s, c
     hipLaunchKernelGGL(kern, dim3((nvec + DEQ_U * 256 - 1) / (DEQ_U * 256)), dim3(256), 0, st, (const uint16_t*)x, nvec,
                        m, sp.ptr, sp.dtype, (const uint16_t*)zp.ptr, f, (uint16_t*)out);
   };
+  vh::note_kernel("k_dequantize_blocks");
   const bool steps = kin == K_STEPS;
   if (m.kind == BLK_SCALAR) steps ? go(k_dequantize_blocks<BLK_SCALAR, false, true>) : go(k_dequantize_blocks<BLK_SCALAR, false, false>);
   else if (m.kind == BLK_ROWS && zp.ptr) go(k_dequantize_blocks<BLK_ROWS, true, false>);
@@ -1456,6 +1461,7 @@ extern "C" int vh_dequantize(const void* x, int32_t x_dtype, const int64_t* shap
     const int64_t n16 = n / 16;
     int64_t blocks = (n16 + 1023) / 1024;
     if (blocks > 4096) blocks = 4096;
+    vh::note_kernel("k_dequantize_tab");
     return dispatch_kind(kernel_kind(fmt_in), [&](auto kind) {
       constexpr int K = decltype(kind)::value;
       if constexpr (K == K_NONE || K == K_IDENTITY || K == K_LUT) {
@@ -1473,6 +1479,7 @@ extern "C" int vh_dequantize(const void* x, int32_t x_dtype, const int64_t* shap
   int64_t threads = (n + VEC - 1) / VEC;
   int64_t blocks = (threads + 255) / 256;
   VH_REQUIRE(blocks < (1ll << 31), "vh_dequantize: tensor too large");
+  vh::note_kernel("k_dequantize");
   return dispatch_kind(kernel_kind(fmt_in), [&](auto kind) {
     constexpr int K = decltype(kind)::value;
     hipLaunchKernelGGL(k_dequantize<K>, dim3((unsigned)blocks), dim3(256), 0, st, x, x_dtype, n, s, sp, zp,

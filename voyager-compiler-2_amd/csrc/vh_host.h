@@ -17,6 +17,9 @@ void set_error(const char* fmt, ...);
 // Check the launch that was just issued; returns VH_OK or VH_ELAUNCH.
 int check_launch(const char* what);
 
+// Records which of its kernels a call launches (vh_last_kernel).
+void note_kernel(const char* name);
+
 inline hipStream_t as_stream(vh_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 inline int dtype_size(int dt) {

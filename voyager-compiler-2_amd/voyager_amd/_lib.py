@@ -96,6 +96,7 @@ _F32 = ctypes.c_float
 
 _SIGNATURES = {
     "vh_last_error": ([], ctypes.c_char_p),
+    "vh_last_kernel": ([], ctypes.c_char_p),
     "vh_abi_version": ([], _I32),
     "vh_build_table": ([ctypes.POINTER(Format), _P, _P], _I32),
     "vh_quantize": (
