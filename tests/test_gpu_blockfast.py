@@ -140,3 +140,17 @@ def test_dequantize_layouts(shape, axis):
         assert _ran() == "k_dequantize"
         assert ran == ("k_dequantize_blocks" if shape[-1] % 8 == 0 else "k_dequantize"), args[2:]
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), args[2:]
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3])
+def test_few_affine_rows(rows):
+    """A token or two into a cache's column blocks, on the general kernel."""
+    q = torch.ops.quantized_ops
+    form = FORMS[8]
+    tab, stab, mid, _ = _tables(form[0], form[3])
+    x = torch.randn(3, rows, 128, generator=torch.Generator().manual_seed(rows)).bfloat16().cuda()
+    got = _quantize(q, x, -2, form, tab, stab, mid)
+    assert _ran() == ("k_cols" if rows <= 2 else "k_fast_cols")
+    ctab, cstab, _, _ = _tables(form[0], form[3], "cpu")
+    for a, b, what in zip(got, _quantize(O, x.cpu(), -2, form, ctab, cstab, None), ("scale", "zero point", "codes")):
+        assert_same_bits(a, b, what)

@@ -489,7 +489,9 @@ int dispatch_scale(const Params& P, F&& fn) {
 // The kernels of vh_blockfast.h, for the forms they take: bf16 tensors,
 // 16-byte aligned, of fewer than 2**31 elements, to bf16 codes and scales,
 // where the row kernel's layout holds, or blocks of 16, 32 or 64 along another
-// dimension with a multiple of eight elements inside it.
+// dimension with a multiple of eight elements inside it.  Affine columns of one
+// or two elements do not pay for the waves' meeting (8 x 1 x 128 in blocks of
+// 32: 5.4 us, 4.5 by k_cols; four elements 5.9, 6.7).
 bool launch_fast(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t block, const Params& P,
                  void* scale_out, void* zp_out, void* codes_out, bool rows_ok, hipStream_t stream) {
   auto al = [](const void* p, int n) { return ((uintptr_t)p & (uintptr_t)(n - 1)) == 0; };
@@ -512,7 +514,8 @@ bool launch_fast(const void* x, int64_t outer, int64_t L, int64_t inner, int64_t
                            make_fast_div((uint32_t)(nblk * g)), g, P, sp, zp, cp);
     });
   }
-  if (inner % 8 || (block != 16 && block != 32 && block != 64) || !al(scale_out, 4) || (zp_out && !al(zp_out, 4)))
+  if (inner % 8 || (block != 16 && block != 32 && block != 64) || !al(scale_out, 4) || (zp_out && !al(zp_out, 4)) ||
+      (P.mode == AFFINE && L <= 2))
     return false;
   const uint32_t total = (uint32_t)(outer * nblk * (inner / 8));
   return dispatch_fast(P, [&](auto m, auto k, auto s) {
