@@ -159,3 +159,15 @@ def test_fp8_scale_of_more_dims_is_refused(rows):
     scale = torch.ones(1, 1, 1, dtype=torch.bfloat16, device="cuda")
     with pytest.raises(ValueError, match="more dims"):
         lower.lowered_fp8_linear(x, scale, formats.quantization_map("fp8_e4m3"), w, scale.reshape(()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rows8_scale_dtypes(dtype):
+    """The E4M3 linear of at most 8 rows under a scale of its own precision:
+    the codes of ``quantize``, whose quotient takes the scale as it is."""
+    x, w = _inputs(7, 48, 1040)
+    tab = formats.quantization_map("fp8_e4m3")
+    sx, one = torch.tensor(0.0137, dtype=dtype, device="cuda"), torch.ones((), dtype=torch.bfloat16, device="cuda")
+    wq = packed.quantize_packed(w, torch.tensor(0.013, dtype=torch.bfloat16, device="cuda"), tab)
+    two = gemm.linear_fp8(packed.quantize_packed(x, sx, tab), wq, one, tile_hint=gemm.TILE_SKINNY)
+    assert torch.equal(gemm.linear_fp8_rows8(x, sx, wq, one), two)

@@ -410,9 +410,14 @@ def linear_mxint8(x_codes, x_scale, w_codes, w_scale, block_size: int, bias_x: i
 def mxint8_two_pass_pays(M: int, N: int, K: int) -> bool:
     """Whether ``linear_mxint8`` rebases both operands to fp16 rows and runs
     the fp16 GEMM rather than decoding the codes in the GEMM's staging.
-    Measured on MI355X (packed / two-pass, us): (K, N) = (4096, 4096) at
-    M = 1024: 53.8 / 60.4, M = 2048: 87.0 / 76.7; (4096, 14336): 161.4 /
-    134.9, 326.1 / 241.6; (14336, 4096): 181.4 / 164.8, 288.8 / 240.3."""
+    Measured on MI355X, whole lowered linears (packed / two-pass, us): (K, N)
+    = (4096, 14336) at M = 1024: 187 / 150, M = 2048: 351 / 252; (14336, 4096):
+    203 / 158, 322 / 241; (4096, 4096) at M = 2048: 108 / 84.1.  Smaller
+    products would gain as well ((4096, 4096) at M = 513 / 1024 / 1536: 58.2 /
+    47.9, 68.2 / 54.7, 102 / 73.8), but the fp16 rows flush blocks more than 24
+    binades under their row's largest, which the packed kernel keeps: the
+    line stays where it has been, and moves with an operand form that does
+    not."""
     return M >= MXI8_TWO_PASS_MIN_M and M * N * K >= MXI8_TWO_PASS_MIN_WORK
 
 
