@@ -43,6 +43,12 @@ def test_direct_tiles(fmt, M, N, K, tile):
     assert _plan(fmt, M, N, K) == (family, tile)
 
 
+@pytest.mark.parametrize("batch,M,N,K", [(256, 17, 1024, 128), (256, 65, 1024, 64), (32, 17, 4096, 64),
+                                         (256, 128, 512, 128)])
+def test_direct_tiles_short_batches(batch, M, N, K):
+    assert _plan(gemm.OP_BF16, M, N, K, batch)[1] == 41
+
+
 @pytest.mark.parametrize("M,N,K,tile", [(2500, 14336, 256, 7), (8192, 8960, 512, 7), (4096, 8960, 256, 7),
                                         (1111, 4096, 14336, 5), (2048, 4096, 4096, 3), (2048, 14336, 4096, 7)])
 def test_fp16_row_tiles(M, N, K, tile):

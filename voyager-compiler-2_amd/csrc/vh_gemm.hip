@@ -2529,7 +2529,10 @@ int staged_tile(int c) {
 // over those sizes (995 of each type) was 1.1% above the best tile (fp8; bf16
 // 1.5%) and up to 47%, now 0.2% (0.4%) and 14% (18%), one bf16 size of K = 256
 // apart (M = 8192, N = 1024: 42%).  fp8 at K = 512, M = 4096, N = 2816 / 14336
-// 23.6 / 78.8 -> 16.0 / 66.8 us.
+// 23.6 / 78.8 -> 16.0 / 66.8 us.  bf16's are fitted to batches as well (2094 of
+// 1 .. 256 products, M = 1 .. 1024, N = 64 .. 4096, K = 64 .. 1024: 0.6% above
+// the best tile, 1.3% as fitted to single products alone, 6.6% by thresholds on
+// the tile counts): 256 products of 17 x 1024 x 128 36.1 -> 31.9 us.
 struct DlTile {
   int tile, bm, bn;
   float f, c0, e, c1;
@@ -2540,9 +2543,9 @@ constexpr DlTile DL_FP8[] = {
     {26, 256, 160, 9.3f, 23.2f, 0.4f, 12.6f}, {44, 256, 224, 9.9f, 41.0f, 2.4f, 11.2f},
     {41, 256, 256, 8.6f, 42.1f, 3.1f, 15.6f}};
 constexpr DlTile DL_BF16[] = {
-    {35, 128, 64, 3.5f, 17.2f, 0.0f, 3.4f},   {33, 128, 128, 4.8f, 21.2f, 0.0f, 10.3f},
-    {25, 128, 192, 6.1f, 27.8f, 0.3f, 15.9f}, {31, 256, 128, 6.6f, 33.1f, 0.9f, 21.6f},
-    {26, 256, 160, 7.5f, 40.0f, 1.1f, 24.6f}, {41, 256, 256, 5.0f, 85.0f, 5.7f, 23.2f}};
+    {35, 128, 64, 3.5f, 17.2f, 0.0f, 3.4f},   {33, 128, 128, 4.5f, 21.2f, 0.3f, 10.3f},
+    {25, 128, 192, 5.4f, 27.8f, 0.4f, 15.9f}, {31, 256, 128, 6.0f, 33.1f, 0.2f, 21.6f},
+    {26, 256, 160, 6.9f, 40.0f, 0.1f, 24.6f}, {41, 256, 256, 4.9f, 85.0f, 2.3f, 23.2f}};
 
 float dl_us(const DlTile& t, int64_t M, int64_t N, int64_t K, int64_t batch) {
   const float k = K < 4096 ? (float)K / 4096.0f : 1.0f, more = K > 4096 ? (float)K / 4096.0f : 1.0f;
