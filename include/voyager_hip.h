@@ -430,9 +430,13 @@ int vh_gemm_nf4_bf16(const uint16_t* x, int64_t M, const uint8_t* w_packed, cons
                      const vh_epilogue* epi, void* y, int64_t ldy, int32_t splits, float* part,
                      int64_t part_bytes, vh_stream_t stream);
 int vh_gemm_nf4_bf16_plan(int64_t M, int64_t N, int64_t K, int32_t* splits);
-/* 1 where decoding both operands once (vh_nf4_decode_bf16) and the bf16 GEMM
- * of vh_gemm is estimated faster than vh_gemm_nf4_bf16, else 0. */
-int vh_gemm_nf4_two_pass(int64_t M, int64_t N, int64_t K);
+/* The form of a linear of these operands estimated fastest: vh_gemm_nf4_bf16,
+ * both operands decoded once (vh_nf4_decode_bf16) and the bf16 GEMM of vh_gemm,
+ * or vh_gemm_nf4. */
+#define VH_NF4_BF16 0
+#define VH_NF4_TWO_PASS 1
+#define VH_NF4_FUSED 2
+int vh_gemm_nf4_route(int64_t M, int64_t N, int64_t K);
 /* Its activation in one pass: quantize_mx of x [M, K] (bfloat16 rows, blocks
  * of 64 along K, minifloat scale map, index table of at most 16 levels), out
  * = bf16(level * scale) -- vh_quantize_mx to index and scale bytes, then

@@ -111,6 +111,17 @@ def test_nf4_two_pass(two, M, N, K):
     assert gemm.nf4_two_pass_pays(M, N, K) == two
 
 
+# (M, N, K) of few blocks of K: the fastest of the three forms
+SHORT = {gemm.NF4_TWO_PASS: [(600, 4608, 64), (256, 256, 256), (201, 4096, 512), (769, 4096, 128), (288, 16400, 1024)],
+         gemm.NF4_FUSED: [(256, 4096, 64), (64, 32768, 256), (201, 32768, 512), (256, 24576, 1024), (400, 7168, 256)],
+         gemm.NF4_BF16: [(160, 11008, 512), (17, 32768, 512), (64, 24576, 1024), (201, 14336, 4096)]}
+
+
+@pytest.mark.parametrize("route,M,N,K", [(r,) + c for r, cs in SHORT.items() for c in cs])
+def test_nf4_route(route, M, N, K):
+    assert load().vh_gemm_nf4_route(M, N, K) == route
+
+
 @pytest.mark.parametrize("N,full", [(64, True), (16384, True), (16400, False), (20480, False), (28672, False),
                                     (32768, True), (32832, False), (65536, True), (128256, True)])
 def test_one_launch_rounds(N, full):

@@ -2919,21 +2919,47 @@ extern "C" int vh_gemm_nf4_bf16_plan(int64_t M, int64_t N, int64_t K, int32_t* s
   return VH_OK;
 }
 
-extern "C" int vh_gemm_nf4_two_pass(int64_t M, int64_t N, int64_t K) {
-  // One row tile covers up to 256 rows; past four of them the bf16 GEMM's
-  // twice as high rate always wins.  Between, both forms by estimate, fitted in
-  // us to whole linears of M = 257 .. 1024, K >= 1024, N = 256 .. 32768 (the
-  // table in voyager_amd/gemm.py): the choice is 0.7% above the better form on
-  // average over 1311 of them; by rows and columns alone, as before, 6.1%.
-  if (M <= 256 || M > 1024 || N < 1 || K < 64) return M > 256;
+extern "C" int vh_gemm_nf4_route(int64_t M, int64_t N, int64_t K) {
+  // Each form's time of a whole linear by estimate, least-squares fits in us on
+  // MI355X (the tables in voyager_amd/gemm.py).  Above 256 rows
+  // vh_gemm_nf4_bf16 decodes a weight block more than once, and past 1024 the
+  // bf16 GEMM's twice as high rate always wins.  Fitted to M = 257 .. 1024,
+  // K >= 1024, N = 256 .. 32768, the choice of the two is 0.7% above the better
+  // one on average over 1311 sizes; by rows and columns alone 6.1%.
+  if (M < 1 || N < 1 || K < 64) return VH_NF4_FUSED;
+  if (M > 1024) return VH_NF4_TWO_PASS;
+  if (M <= 256 && K > 1024) return VH_NF4_BF16;
   const Nf4bPlan p = nf4b_plan(M, N, K, 0);
-  const float h = (float)p.bm / 64.0f, groups = (float)p.tiles * (float)p.splits;
+  const float h = (float)p.bm / 64.0f, full = (float)p.tiles * (float)p.splits / 256.0f;
   const float rounds = (float)((p.tiles * p.splits + 255) / 256);
   const float mn = (float)M * (float)N * 1e-6f, nk = (float)N * (float)K * 1e-6f;
-  const float one = 7.9f + rounds * (p.kcs * (0.202f + 0.075f * h) + 2.38f * h) + groups / 256.0f * p.kcs * 0.047f * h +
-                    (p.splits > 1 ? 1.97f * p.splits * mn : 0.0f);
-  const float two = 11.3f + 0.514f * nk + 1.07f * dl_us(dl_tile(DL_BF16, M, N, K, 1), M, N, K, 1);
-  return one > two;
+  const float dl = dl_us(dl_tile(DL_BF16, M, N, K, 1), M, N, K, 1);
+  if (K > 1024) {
+    const float one = 7.9f + rounds * (p.kcs * (0.202f + 0.075f * h) + 2.38f * h) + full * p.kcs * 0.047f * h +
+                      (p.splits > 1 ? 1.97f * p.splits * mn : 0.0f);
+    return one > 11.3f + 0.514f * nk + 1.07f * dl ? VH_NF4_TWO_PASS : VH_NF4_BF16;
+  }
+  // Few blocks of K: launches, fills and stores weigh more, and vh_gemm_nf4,
+  // with half as many workgroups to set up, is the fastest of the three for the
+  // shortest and widest.  Fitted to K = 64 .. 1024, N = 256 .. 32768, 17 .. 1024
+  // rows: 1.3% above the fastest of the three on average over 2976 sizes; by
+  // thresholds on M, N and K 3.5%.
+  const float one = 5.8f + rounds * (3.57f + 0.095f * p.kcs) + full * p.kcs * h * 0.162f + rounds * h * 1.87f +
+                    (p.splits > 1 ? 0.24f + 1.15f * p.splits * mn : 0.0f);
+  const float two = 6.4f + 0.768f * nk + 1.335f * dl;
+  if (M < 512) {
+    int32_t tile = 0, splits = 0;
+    int64_t bm = 0;
+    if (vh_gemm_nf4_plan(M, N, K, &tile, &splits, &bm) != VH_OK) return VH_NF4_FUSED;
+    const int64_t groups = (M + bm - 1) / bm * ((N + 127) / 128) * splits;
+    const float kcs = (float)((K / 64 + splits - 1) / splits), r = (float)((groups + 255) / 256);
+    const float f = (float)groups / 256.0f;
+    const float fused = 9.5f + (tile == 2 ? r * (2.65f + 1.446f * kcs) + f * 0.126f * kcs
+                                          : r * (0.73f + 0.385f * kcs) + f * 0.875f * kcs) +
+                        (splits > 1 ? 2.97f + 1.6f * splits * mn : 0.0f);
+    if (fused < one && fused < two) return VH_NF4_FUSED;
+  }
+  return two < one ? VH_NF4_TWO_PASS : VH_NF4_BF16;
 }
 
 extern "C" int vh_gemm_nf4_bf16(const uint16_t* x, int64_t M, const uint8_t* w_packed, const uint8_t* w_scale,

@@ -155,7 +155,7 @@ _SIGNATURES = {
     "vh_gemm_nf4_bf16": ([_P, _I64, _P, _P, ctypes.POINTER(Format), _P, _I64, _I64, _P, _P, _I64, _I32, _P, _I64,
                           _P], _I32),
     "vh_gemm_nf4_bf16_plan": ([_I64, _I64, _I64, _P], _I32),
-    "vh_gemm_nf4_two_pass": ([_I64, _I64, _I64], _I32),
+    "vh_gemm_nf4_route": ([_I64, _I64, _I64], _I32),
     "vh_nf4_quantize_bf16": ([_P, _I64, _I64, ctypes.c_float, ctypes.POINTER(Format), ctypes.POINTER(Format), _P,
                               _P, _P], _I32),
     "vh_nf4_decode_bf16": ([_P, _P, ctypes.POINTER(Format), _I64, _P, _P, ctypes.POINTER(Format), _P, _I64, _I64,

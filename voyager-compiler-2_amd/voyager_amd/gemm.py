@@ -695,21 +695,29 @@ def linear_nf4_prefill(x: torch.Tensor, weight: NF4Weight, index_table: torch.Te
 
 
 def _nf4_route(M: int, weight: NF4Weight) -> str:
-    """The kernels of an MXNF4 prefill: "two" (``nf4_two_pass_pays``), "bf16"
-    (``vh_gemm_nf4_bf16``) or "fused" (``vh_gemm_nf4``): where the weight does
-    not lie as the second's loads need, and for short K, whose few blocks do
-    not pay for its setup (M = 256, K = 64: 17.6 us against 10.7; K = 512, N =
-    14336, M = 300: 29.4 against 23.8, K = 1024 37.4 against 36.7)."""
-    N, K = weight.N, weight.K
-    if nf4_two_pass_pays(M, N, K):
-        return "two"
-    fits = K <= 1 << 20 and weight.packed.data_ptr() % 16 == 0 and weight.scale.data_ptr() % 16 == 0
-    return "bf16" if M >= 1 and fits and not _nf4_short(M, N, K) else "fused"
+    """The kernels of an MXNF4 prefill, by ``vh_gemm_nf4_route``'s estimate:
+    "two" (``nf4_two_pass_pays``), "bf16" (``vh_gemm_nf4_bf16``) or "fused"
+    (``vh_gemm_nf4``), the last also where the weight does not lie as the
+    second's loads need.  Few blocks of K do not pay for the setup of the
+    second, a column strip of all rows in each workgroup.  Measured on MI355X,
+    whole linears, us (``vh_gemm_nf4_bf16`` / two-pass / ``vh_gemm_nf4``):
+
+    (K, N)         M = 64                201                   256                   400
+    (64, 4096)     12.0  11.3  10.7    16.7  11.6  10.8    17.6  11.7  10.8    17.0  12.1  11.1
+    (256, 4096)    12.1  12.3  15.0    16.8  12.6  18.0    17.7  12.7  19.2    17.0  13.1  21.8
+    (512, 14336)   12.6  22.6  22.3    20.6  24.1  20.1    22.6  24.5  20.7    35.2  28.7  24.8
+    (256, 28672)   19.2  21.9  15.8    30.4  26.3  18.1    33.1  27.2  18.8    52.6  29.9  29.5
+    (1024, 24576)  23.6  35.4  33.0    43.7  40.6  35.5    48.0  41.0  36.8    63.5  54.7  65.0
+    """
+    route = load().vh_gemm_nf4_route(M, weight.N, weight.K)
+    if route == NF4_BF16:
+        fits = weight.K <= 1 << 20 and weight.packed.data_ptr() % 16 == 0 and weight.scale.data_ptr() % 16 == 0
+        return "bf16" if fits else "fused"
+    return "two" if route == NF4_TWO_PASS else "fused"
 
 
-def _nf4_short(M: int, N: int, K: int) -> bool:
-    """Too few blocks of K for ``vh_gemm_nf4_bf16`` and the two passes alike."""
-    return M < 512 and (K <= 128 and (M >= 64 or N > 16384) or K < 1024 and N > 8192 and M > 256)
+#: ``vh_gemm_nf4_route``
+NF4_BF16, NF4_TWO_PASS, NF4_FUSED = 0, 1, 2
 
 
 def nf4_quantize_bf16(x: torch.Tensor, weight: NF4Weight, ec, sc) -> torch.Tensor:
@@ -760,10 +768,10 @@ def nf4_two_pass_pays(M: int, N: int, K: int) -> bool:
 
     Up to 256 rows the one tile of rows decides.  Above, a row costs the first
     more and the weight's decode, which grows with K and N, is saved once;
-    both in rounds of the CUs, so ``vh_gemm_nf4_two_pass`` compares the two by
-    estimate.  The two-pass form holds the decoded weight (2 bytes per
+    both in rounds of the CUs, so ``vh_gemm_nf4_route`` compares them by estimate.
+    The two-pass form holds the decoded weight (2 bytes per
     element) for the call."""
-    return not _nf4_short(M, N, K) and bool(load().vh_gemm_nf4_two_pass(M, N, K))
+    return load().vh_gemm_nf4_route(M, N, K) == NF4_TWO_PASS
 
 
 def gemm_nf4_packed(px, weight: NF4Weight, out_dtype=torch.bfloat16, bias=None, alpha=None, tile: int = 0,
