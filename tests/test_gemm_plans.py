@@ -78,6 +78,8 @@ def test_few_rows(fmt, few, M, N, K, batch):
     assert (_plan(fmt, M, N, K, batch)[0] == gemm.FAMILY_SKINNY) == few
     if M <= 64:
         assert _plan(fmt, M, N, K, batch, gemm.TILE_SKINNY)[0] == gemm.FAMILY_SKINNY
+    else:  # as any hint that names no tile of its own
+        assert _plan(fmt, M, N, K, batch, gemm.TILE_SKINNY) == (gemm.FAMILY_STAGED, 4)
 
 
 @pytest.mark.parametrize("fmt", [gemm.OP_BF16, gemm.OP_FP8, gemm.OP_MXI8])

@@ -132,6 +132,15 @@ def test_skinny_bf16(M, N, K, out_dtype):
     assert max_rel_err(yb, torch.stack([ref, ref])) < room
 
 
+def test_skinny_hint_past_its_rows():
+    """A hint for the few-row kernel runs the tiles where it cannot."""
+    x, w = _inputs(65, 136, 320)
+    x = x.clamp(-8, 8)
+    y, log = _log(lambda: gemm.gemm_bf16(x, w, torch.float32, tile_hint=gemm.TILE_SKINNY))
+    assert [p[0] for p in log] == [gemm.FAMILY_STAGED]
+    assert max_rel_err(y, x.double() @ w.double().T) < 1e-5
+
+
 def test_rows8_nan_and_infinity():
     """Values the fast quotients do not decide: NaN, infinities, quotients on
     a bf16 rounding midpoint, in one launch as in two."""

@@ -2655,8 +2655,6 @@ extern "C" int vh_gemm(const vh_gemm_desc* d, vh_stream_t stream) {
     if (fmt == OP_P8) VH_REQUIRE(d->lut, "vh_gemm: posit8 operand needs its decode table");
   }
   VH_REQUIRE(d->lda * 256 < (1ll << 31) && d->ldb * 256 < (1ll << 31), "vh_gemm: rows too long for 32-bit offsets");
-  VH_REQUIRE(d->tile_hint != VH_GEMM_TILE_SKINNY || vh::skinny_fits(d),
-             "vh_gemm: the few-row kernel cannot take this product");
   if (d->M == 0 || d->N == 0) return VH_OK;
   GemmArgs g;
   memset(&g, 0, sizeof(g));

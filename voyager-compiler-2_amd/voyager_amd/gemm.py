@@ -59,7 +59,7 @@ class GemmDesc(ctypes.Structure):
 
 
 FAMILY_STAGED, FAMILY_DIRECT_FP8, FAMILY_DIRECT_BF16, FAMILY_MXI8, FAMILY_SKINNY = 1, 2, 3, 4, 5
-TILE_SKINNY = 70  # the few-row kernel, whatever the rule of vh_gemm says
+TILE_SKINNY = 70  # the few-row kernel where it can run, whatever the rule of vh_gemm says
 
 #: When set to a list, every ``vh_gemm`` launch appends ``(family, tile,
 #: splits, M, N, K)`` of the kernel it runs (``vh_gemm_plan``), so tests can
