@@ -110,3 +110,21 @@ def test_linear_nf4_routes(form, M, K, N):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, call())
+
+
+@pytest.mark.parametrize("M,K,N", [(201, 256, 1040), (600, 512, 272)])
+def test_given_tile_runs_the_fused_kernel(M, K, N):
+    """Where two passes are the choice, a given tile or split still runs
+    ``vh_gemm_nf4`` at it."""
+    from voyager_amd import gemm, packed
+
+    index, entries, stab = _maps()
+    g = torch.Generator().manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    wb = gemm.bake_nf4_weight((torch.randn(N, K, generator=g) * 0.02).bfloat16().cuda(), index, stab, entries)
+    assert gemm.nf4_two_pass_pays(M, N, K)
+    px = packed.quantize_mx_packed(x, index, [-1], 64, 31.0, False, stab)
+    for tile, splits in ((1, 1), (2, 0), (0, 2)):
+        ref = gemm.linear_nf4_prefill(x, wb, index, stab, torch.float32, tile=tile, splits=splits, two_pass=False)
+        assert torch.equal(gemm.gemm_nf4_packed(px, wb, torch.float32, tile=tile, splits=splits), ref)
+        assert torch.equal(gemm.linear_nf4_prefill(x, wb, index, stab, torch.float32, tile=tile, splits=splits), ref)

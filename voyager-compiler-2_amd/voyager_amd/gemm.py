@@ -766,11 +766,11 @@ def nf4_two_pass_pays(M: int, N: int, K: int) -> bool:
     (4096, 14336)  61.4 / 74.8  85.8 / 92.4   102 / 98.0   115 / 102    163 / 137    219 / 157
     (14336, 4096)  58.9 / 107   72.5 / 113   89.4 / 121    105 / 131    167 / 155    186 / 177
 
-    Up to 256 rows the one tile of rows decides.  Above, a row costs the first
-    more and the weight's decode, which grows with K and N, is saved once;
-    both in rounds of the CUs, so ``vh_gemm_nf4_route`` compares them by estimate.
-    The two-pass form holds the decoded weight (2 bytes per
-    element) for the call."""
+    Up to 256 rows (few blocks of K aside, ``_nf4_route``) the one tile of rows
+    decides.  Above, a row costs the first more and the weight's decode, which
+    grows with K and N, is saved once; both in rounds of the CUs, so
+    ``vh_gemm_nf4_route`` compares them by estimate.  The two-pass form holds
+    the decoded weight (2 bytes per element) for the call."""
     return load().vh_gemm_nf4_route(M, N, K) == NF4_TWO_PASS
 
 
@@ -788,9 +788,9 @@ def gemm_nf4_packed(px, weight: NF4Weight, out_dtype=torch.bfloat16, bias=None, 
     if K != weight.K:
         raise RuntimeError("gemm_nf4_packed: contraction mismatch")
     if two_pass is None:
-        route = _nf4_route(M, weight)
+        route = _nf4_route(M, weight) if tile == 0 and splits == 0 else "fused"
         two_pass = route == "two"
-        if tile == 0 and splits == 0 and route == "bf16":
+        if route == "bf16":
             xo, _ = nf4_decode_bf16(px, weight, decode_w=False)
             return gemm_nf4_bf16(xo, weight, out_dtype, bias, alpha)
     if two_pass:
