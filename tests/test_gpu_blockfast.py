@@ -2,9 +2,9 @@
 (``vh_blockfast.h``, ``k_dequantize_blocks``) against the general kernels, bit
 for bit and with the kernel that ran asserted: the same values behind a 16-byte
 aligned address, which they need, and behind one that is not, over every form
-they take, at edges of blocks, rows and workgroups, with zeros, NaN, infinities, subnormal and huge blocks, quotients on
-rounding midpoints and scales that saturate or flush their map; a case of each
-against the oracle."""
+they take, at edges of blocks, rows and workgroups, with zeros, NaN, infinities,
+subnormal and huge blocks, quotients on rounding midpoints and scales that
+saturate or flush their map; a case of each against the oracle."""
 
 import pytest
 import torch
